@@ -31,7 +31,7 @@ SOURCES = [
     "kernels/qmm.hip",
     "kernels/qmm_wide.hip",
     "kernels/qmm_dma.hip", "kernels/qmm_small.hip",
-    "kernels/qmm_n.hip",
+    "kernels/qmm_n.hip", "kernels/qmm_tile_n.hip",
     "kernels/gather.hip",
     "kernels/gather_decode.hip", "kernels/qmm_rows.hip",
     "kernels/moe.hip",

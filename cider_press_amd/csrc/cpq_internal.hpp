@@ -90,12 +90,21 @@ struct QuantArgs {
 };
 
 hipError_t launch_dequantize(hipStream_t s, const QuantArgs& q, void* out, size_t n_out);
-// Y[M, N] = X[M, K] . dequant(W[K, N]) (MLX transpose=false); N % 32 == 0,
-// K % 8 == 0.  split > 1 splits K and needs qmm_n_scratch_bytes of fp32 partials.
-int qmm_n_split(int m, int n, int k, int cu_count);
-size_t qmm_n_scratch_bytes(int m, int n, int split);
-hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
-                        float* partial);
+// A tile size (an index into its direction's table), the K split, the scratch
+// that takes and the estimated time.  cfg < 0: the shape is not supported.
+struct TilePlan {
+  int cfg;
+  int split;
+  size_t scratch_bytes;
+  float us;
+};
+// Y[M, N] = X[M, K] . dequant(W[K, N]) (MLX transpose=false) on tiles, every
+// width; N % 32 == 0, K % 8 == 0, K > 0, tables within 31-bit byte offsets.
+TilePlan qmm_tile_n_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
+hipError_t launch_qmm_tile_n(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,
+                             void* y, int m, int n, int k);
+// The same for what the tiles do not take: K = 0 (stores zeros), larger tables.
+hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
 // Decode (M = 1) transpose=false at 4/8 bits on the VALU: rows per thread
 // and step, K parts and the split-K scratch they need (arrival words at the
 // head, zero between launches, then fp32 sums); parts == 1 needs none.
