@@ -816,7 +816,7 @@ TRACE_WORKLOADS = (
     ("qmm_dma_kernel", 196608, "cfg3b"),
     ("qmm_dma_kernel", 262144, "cfg3c N=4096"),
     ("qmm_dma_kernel", 786432, "cfg3c N=12288"),
-    ("qmm_staged_kernel<cpq::dev::BF16, 8", 65536, "8-bit prefill M=512"),
+    ("qmm_tile_t_kernel<cpq::tile::TCfg<cpq::dev::BF16, 8", 65536, "8-bit prefill M=512"),
     ("qmv_lean_kernel<cpq::dev::BF16, 4, 6, 4, 8, true, false>", 65536, "cfg4 4b gs64 M=1"),
     ("qmv_lean_kernel<cpq::dev::BF16, 4, 5, 4, 8, true, false>", 65536, "cfg4 4b gs32 M=1"),
     ("qmv_lean_kernel<cpq::dev::BF16, 8, 6, 4, 8, true, false>", 65536, "cfg4 8b M=1"),

@@ -29,7 +29,7 @@ SOURCES = [
     "kernels/qmv.hip",
     "kernels/skinny.hip",
     "kernels/qmm.hip",
-    "kernels/qmm_wide.hip",
+    "kernels/qmm_tile_t.hip",
     "kernels/qmm_dma.hip", "kernels/qmm_small.hip",
     "kernels/qmm_n.hip", "kernels/qmm_tile_n.hip",
     "kernels/gather.hip",

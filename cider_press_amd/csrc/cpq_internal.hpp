@@ -103,7 +103,12 @@ struct TilePlan {
 TilePlan qmm_tile_n_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
 hipError_t launch_qmm_tile_n(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,
                              void* y, int m, int n, int k);
-// The same for what the tiles do not take: K = 0 (stores zeros), larger tables.
+// Y[M, N] = X[M, K] . dequant(W[N, K])^T on tiles, every width; N % 32 == 0,
+// K <= 2^21.
+TilePlan qmm_tile_t_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
+hipError_t launch_qmm_tile_t(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,
+                             void* y, int m, int n, int k);
+// transpose=false for what its tiles do not take: K = 0 (stores zeros), larger tables.
 hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
 // Decode (M = 1) transpose=false at 4/8 bits on the VALU: rows per thread
 // and step, K parts and the split-K scratch they need (arrival words at the
@@ -171,11 +176,12 @@ hipError_t launch_qmm_skinny(hipStream_t s, const QuantArgs& q, const void* x, v
 // the CU count and the capacity of the scratch the caller can give it;
 // launch_qmm runs that plan, with `scratch` holding at least
 // plan.scratch_bytes (arrival counters zeroed) when that is nonzero.
-enum class QmmKernel { Unsplit, Wide, Dma };
+enum class QmmKernel { Unsplit, Tile, Dma };
 struct QmmPlan {
-  QmmKernel kernel;      // Dma / Wide (4-bit, K split possible) or a kernel that needs no scratch
+  QmmKernel kernel;      // Dma / Tile (K split possible) or the kernel that needs no scratch
   int split;             // its K split
   size_t scratch_bytes;  // scratch the plan uses (0: none)
+  TilePlan tile;         // of a Tile plan
 };
 QmmPlan qmm_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
 hipError_t launch_qmm(hipStream_t s, const QmmPlan& plan, void* scratch, const QuantArgs& q, const void* x,
@@ -202,27 +208,20 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
 // Capacity of a session's scratch when CPQ_SESSION_SCRATCH_MB is not set.
 constexpr size_t kDefaultSessionScratchBytes = size_t(64) << 20;
 
-// Prefill kernels that need no session scratch (staged, streaming or the
-// LDS-tiled fallback, by shape); any M, K, group size and width.
+// The general prefill kernel: no session scratch, any M, N, K, group size and
+// width.
 hipError_t launch_qmm_unsplit(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
 
-// Wide-tile prefill kernel (4-bit, 128 x 128 tiles, optional split K).
 constexpr size_t kWideCounterBytes = 64 * 1024;  // arrival counters at the head of the scratch
-bool qmm_wide_fits(int m, int n, int k, int gs, int bits, int split);
-// Split (1, 2 or 4) that minimises the estimated makespan; 0 if the kernel
-// does not apply.
-int qmm_wide_split(int m, int n, int k, int gs, int bits, int cu_count);
-size_t qmm_wide_scratch_bytes(int m, int n, int split);
-hipError_t launch_qmm_wide(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n,
-                           int k, int split, void* scratch);
 hipError_t zero_words(hipStream_t s, void* p, size_t n_words);
 
 // Prefill kernel with two waves per SIMD (4-bit, 128 x 128 tiles, both
-// operands streamed into LDS, optional split K; same scratch layout as the
-// wide kernel: arrival counters, then fp32 partial tiles).
+// operands streamed into LDS, optional split K; scratch: arrival counters, then
+// fp32 partial tiles).
 bool qmm_dma_fits(int m, int n, int k, int gs, int bits, int split);
 int qmm_dma_split(int m, int n, int k, int gs, int bits, int cu_count);
 size_t qmm_dma_scratch_bytes(int m, int n, int split);
+float qmm_dma_us(int m, int n, int k, int split, int cu_count);
 hipError_t launch_qmm_dma(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
                           void* scratch);
 

@@ -663,6 +663,16 @@ int qmm_dma_split(int m, int n, int k, int gs, int bits, int cu_count) {
   return best;
 }
 
+// Estimated time: the k-units of the split's makespan at 6.1 ns, and for a
+// split 2 us and its parked bytes (written and read, mostly through the L2 of
+// one XCD) at 16 TB/s.
+float qmm_dma_us(int m, int n, int k, int split, int cu_count) {
+  const long tiles = (long)((m + DBM - 1) / DBM) * ((n + DBN - 1) / DBN);
+  const long cus = cu_count > 0 ? cu_count : 256, rounds = (tiles * split + cus - 1) / cus;
+  const float us = 0.0061f * (float)(rounds * (k / split + 2000));
+  return split > 1 ? us + 2.f + 2.f * (float)(tiles * split * DPART * 4) / 16e6f : us;
+}
+
 size_t qmm_dma_scratch_bytes(int m, int n, int split) {
   if (split <= 1) return 0;
   const size_t tiles = (size_t)((m + DBM - 1) / DBM) * ((n + DBN - 1) / DBN);

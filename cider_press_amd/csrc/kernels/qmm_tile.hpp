@@ -1,7 +1,9 @@
 // Tiled quantized GEMM for gfx950, every width and both weight directions.
 //
-//   KN = false:  Y[M,N] = X[M,K] . dequant(W[N,K])^T   (affine_qmm_t)
-//   KN = true:   Y[M,N] = X[M,K] . dequant(W[K,N])     (affine_qmm_n)
+//   qmm_tile_t.hip:  Y[M,N] = X[M,K] . dequant(W[N,K])^T   (affine_qmm_t)
+//   qmm_tile_n.hip:  Y[M,N] = X[M,K] . dequant(W[K,N])     (affine_qmm_n)
+//
+// This file: what both share, and the choice of tile and K split.
 //
 // Reference ops: qmm_t_impl / qmm_n_impl (kernels-mlx/mlx/backend/metal/
 // kernels/quantized.h:1087-1213, 1215-1349).  Numerics as every path here:

@@ -1,9 +1,13 @@
 """The tiled matmul kernels: every tile size and K split forced, at the edges
 of tiles, K stages and groups, every width; scales too large for the
 subnormal form of the dequantization."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from cider_press_amd import _lib
+from cider_press_amd.kernels import _ptr
 from cider_press_amd.kernels import qmm as kqmm
 from cider_press_amd.synthetic import from_bits, make_weight, make_x, to_bits
 
@@ -69,3 +73,88 @@ def test_tile_n_large_scales(device, library, oracle, monkeypatch, split):
     _close(outs[0][:, 64:128], ref[:, 64:128], "bf16")
     rest = np.r_[0:64, 128:512]
     _close(outs[0][:, rest], ref[:, rest], "bf16")
+
+
+def _run_t(device, library, oracle, m, n, k, gs, bits, dtype, edit=None, calls=1, skew=0):
+    """affine_qmm_t and its float64 reference; `skew` starts the scales and
+    biases that many elements into their allocations."""
+    rng = np.random.default_rng(m * 5 + n + k + bits)
+    w_q, s, b = make_weight(rng, n, k, gs, bits, dtype)
+    if edit:
+        edit(s, b)
+    x = make_x(rng, m, k, dtype)
+    W = device.upload(w_q.reshape(-1), "u32")
+    pad = np.zeros(skew, np.uint16)
+    S, B = (device.upload(np.concatenate([pad, t.reshape(-1)]), dtype) for t in (s, b))
+    X = device.upload(x.reshape(-1), dtype)
+    cmds, outs = device.commands(), []
+    for _ in range(calls):
+        Y = device.alloc_buffer(m * n, dtype)
+        at = lambda t: ctypes.c_void_p(t.ptr + 2 * skew)  # noqa: E731
+        _lib.check(_lib.lib().cpq_affine_qmm_t(
+            cmds.handle, _lib.DTYPES[dtype], _ptr(W), len(W), at(S), s.size, at(B), b.size, _ptr(X), len(X), _ptr(Y),
+            len(Y), m, n, k, gs, bits))
+        cmds.commit_and_wait()
+        outs.append(Y.to_numpy().reshape(m, n))
+    w = from_bits(oracle.dequantize(w_q, s, b, n, k, gs, bits, dtype), dtype).astype(np.float64)
+    return outs, from_bits(x, dtype).astype(np.float64) @ w.T
+
+
+@pytest.fixture
+def tiles(monkeypatch):
+    """affine_qmm_t on the tiles at every M."""
+    monkeypatch.setenv("CPQ_QMM_DMA", "0")
+    monkeypatch.setenv("CPQ_SKINNY_MAX_M", "1")
+    monkeypatch.setenv("CPQ_SMALL_ROWS", "0")
+    monkeypatch.setenv("CPQ_SMALL_DENSE", "0")
+    return monkeypatch
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("m,n,k,gs,bits,dtype,split,skew", [
+    (2, 32, 32, 32, 6, "bf16", 1, 0),      # one 32-k stage
+    (257, 288, 96, 32, 4, "bf16", 1, 1),   # one past a tile, K half a stage past one, odd table start
+    (65, 128, 288, 32, 8, "f16", 2, 1),    # 9 groups a row: rows of 2-byte aligned scales
+    (33, 416, 1088, 32, 3, "bf16", 3, 0),  # blocks of 8 groups end inside the parts
+    (129, 384, 1024, 128, 5, "f16", 5, 1),
+    (40, 256, 704, 64, 2, "bf16", 1, 0),   # 11 groups a row
+    (130, 256, 2112, 64, 6, "bf16", 4, 1),
+    (70, 160, 1280, 32, 4, "f16", 7, 0),
+])
+def test_tile_t(device, library, oracle, tiles, cfg, m, n, k, gs, bits, dtype, split, skew):
+    tiles.setenv("CPQ_TILE_CFG", str(cfg))
+    tiles.setenv("CPQ_QMM_SPLIT", str(split))
+    outs, ref = _run_t(device, library, oracle, m, n, k, gs, bits, dtype, calls=2, skew=skew)
+    _close(outs[0], ref, dtype)
+    assert np.array_equal(outs[0], outs[1])
+
+
+def test_tile_t_skips_values_past_k(device, library, oracle, tiles):
+    """The half stage past K holds the next row of X: an infinity there must
+    not reach the row before it."""
+    m, n, k, gs = 40, 64, 96, 32
+    rng = np.random.default_rng(3)
+    w_q, s, b = make_weight(rng, n, k, gs, 4, "bf16")
+    x = make_x(rng, m, k, "bf16")
+    x[7, 3] = 0x7F80
+    W, S, B = (device.upload(t.reshape(-1), d) for t, d in ((w_q, "u32"), (s, "bf16"), (b, "bf16")))
+    X, Y, cmds = device.upload(x.reshape(-1), "bf16"), device.alloc_buffer(m * n, "bf16"), device.commands()
+    kqmm.affine_qmm_t(cmds, library, W, S, B, X, Y, m, n, k, gs, 4)
+    cmds.commit_and_wait()
+    y = from_bits(Y.to_numpy().reshape(m, n), "bf16")
+    assert not np.isfinite(y[7]).any()
+    assert np.isfinite(np.delete(y, 7, axis=0)).all()
+
+
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("value", [2.0 ** 104, 2.0 ** 120])
+def test_tile_t_large_scales(device, library, oracle, tiles, split, value):
+    tiles.setenv("CPQ_QMM_SPLIT", str(split))
+
+    def edit(s, b):
+        s[70, 2] = to_bits(np.float32([value]), "bf16")[0]
+        b[70, 2] = to_bits(np.float32([-2.0 ** 100]), "bf16")[0]
+
+    outs, ref = _run_t(device, library, oracle, 70, 512, 256, 64, 4, "bf16", edit)
+    _close(outs[0][:, [70]], ref[:, [70]], "bf16")
+    _close(np.delete(outs[0], 70, axis=1), np.delete(ref, 70, axis=1), "bf16")
