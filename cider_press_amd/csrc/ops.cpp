@@ -8,6 +8,7 @@
 // Validation order and messages follow those functions so error behaviour is
 // the same; "kernel not found" is reported after shape validation, as the
 // reference's pipeline lookup is (qmv.rs:172-173, library.rs:264-286).
+#include <algorithm>
 #include <climits>
 #include <cstdlib>
 #include <string>
@@ -101,11 +102,38 @@ using cpq::fail;
 
 namespace cpq {
 
+namespace {
+
+// Estimated time (us) of the small-M kernel a shape would run on without the
+// tiles: the dense form (8-row passes; it slows down once the passes' weights
+// pass about 25M), the tiled small-M kernel (rounds of one workgroup per CU,
+// its K range; chunks of it restage activations), or the slab kernel (rounds of
+// 16-column slabs).  Fitted to calls of M = 2 .. 64 at (N, K) from 1152 to 12288;
+// within about 20 % where the choice is close.
+float small_m_us(const QuantArgs& q, const SmallPlan& sp, bool dense, int m, int n, int k, long cus) {
+  const float kf = (float)k / 1024.f;
+  if (dense) {
+    const float v = (float)((m + 7) / 8) * (float)n * (float)k * 1e-6f;
+    return 4.f + 0.13f * std::min(v, 25.f) + 0.33f * std::max(0.f, v - 25.f) + 0.92f * kf;
+  }
+  if (sp.split > 0 && sp.mb == 1) return 4.f + (q.bits == 8 ? 1.8f : 1.2f) * kf * std::max(1.f, (float)n / 4096.f);
+  if (sp.split > 0) {
+    const long wgs = (long)((n + 16 * sp.mb - 1) / (16 * sp.mb)) * sp.split;
+    return 6.f + 1.1f * (float)sp.mb * kf / (float)sp.split * (float)((wgs + cus - 1) / cus) * (sp.nch > 1 ? 1.8f : 1.f) +
+           (sp.split > 1 ? 3.f : 0.f);
+  }
+  const float passes = (float)((m + 15) / 16);
+  return (4.f + 1.9f * kf) * (float)(((n + 15) / 16 + cus - 1) / cus) * (1.f + 0.015f * (float)std::min(m, 16)) *
+         (1.f + 0.4f * (passes - 1.f));
+}
+
+}  // namespace
+
 // Y[M, N] = X[M, K] . W^T on validated operands: the kernel the shape runs
 // best on.  Up to skinny_max_m rows: at K = 4096 / 8192 / 16384 (4/8-bit, up
-// to 16 rows) the decode kernel's layout with M activation rows; other
-// 4/8-bit shapes with K a multiple of 256 the tiled small-M kernel; other
-// shapes the slab kernel.  Larger M: the prefill plan.  Plans are made for
+// to 16 rows) the decode kernel's layout with M activation rows; else one of
+// the other small-M kernels (below) or, where that is estimated to be faster,
+// the prefill tiles.  Larger M: the prefill plan.  Plans are made for
 // ex.plan_bytes of scratch and, when that plan needs more than the
 // ex.scratch_bytes at hand, for ex.scratch_bytes.  CPQ_SMALL_M=0 forces the
 // slab kernel, CPQ_QMV_ROWS=0 skips the decode layout (tuning hooks).
@@ -143,7 +171,22 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
     // kernel (K in 128-element steps split over the waves of a workgroup,
     // 8 rows per workgroup).
     const long small_wgs = sp.split > 0 ? (long)sp.split * ((n + 16 * sp.mb - 1) / (16 * sp.mb)) : 0;
-    if (dense_ok && small_wgs * 4 < cus) return launch_dense_small(ex.stream, q, x, y, m, n, k);
+    const bool dense = dense_ok && small_wgs * 4 < cus;
+    const float est = small_m_us(q, sp, dense, m, n, k, cus);
+    TilePlan tp{-1, 1, 0, 0.f};
+    if (small_on && dense_env < 1 && est > 6.f) {  // no tile takes less
+      tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.plan_bytes);
+      if (tp.scratch_bytes > ex.scratch_bytes) tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
+    }
+    // The tiles where they are estimated to take a good deal less (past 16
+    // rows the dense form repeats its dequantization per 8 rows, a K that does
+    // not split leaves the tiled small-M kernel few workgroups, and the slab
+    // kernel reads each activation slice from L2 per wave): 48 x 4096 x 11008
+    // 102 -> 24 us, 60 x 9984 x 3520 91 -> 18, 24 x 3520 x 3520 14.8 -> 11.5,
+    // 6-bit 16 x 2560 x 10048 29 -> 19; 32 x 4096 x 4096 stays (11.3 / 12.4).
+    if (tp.cfg >= 0 && tp.us < 0.92f * est)
+      return launch_qmm_tile_t(ex.stream, tp, ex.scratch, q, x, y, m, n, k);
+    if (dense) return launch_dense_small(ex.stream, q, x, y, m, n, k);
     if (sp.split > 0) return launch_qmm_small(ex.stream, sp, ex.scratch, q, x, y, m, n, k);
     return launch_qmm_skinny(ex.stream, q, x, y, m, n, k);
   }
