@@ -26,7 +26,7 @@ SOURCES = [
     "noalloc.hip",
     "kernels/dequantize.hip",
     "kernels/embed.hip",
-    "kernels/qmv.hip",
+    "kernels/qmv.hip", "kernels/decode.hip",
     "kernels/skinny.hip",
     "kernels/qmm.hip",
     "kernels/qmm_tile_t.hip",

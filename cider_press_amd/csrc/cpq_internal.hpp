@@ -142,6 +142,12 @@ hipError_t launch_embed(hipStream_t s, const QuantArgs& q, const uint32_t* ids, 
 // Decode GEMV: y[N] = x[K] . W^T for one activation row.
 hipError_t launch_qmv(hipStream_t s, const QuantArgs& q, const void* x, void* y, int n, int k);
 
+// The decode kernel for up to 16 rows at every width (kernels/decode.hip): K a
+// multiple of 32, M * K * 2 bytes and the K parts within LDS, x and w 16-byte
+// aligned.
+bool decode_fits(const QuantArgs& q, int m, int n, int k, const void* x);
+hipError_t launch_decode(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
+
 // A batch folded into a grid dimension (MLX's adjust_matrix_offsets):
 // element z (row-major over shape[0..nd)) takes its operands at
 // sum_d idx_d(z) * st[o][d] elements (o: w_q in u32 words, scales, biases,

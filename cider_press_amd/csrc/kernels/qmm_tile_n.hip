@@ -258,7 +258,7 @@ __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   keep(c1);
 
   // A scale too large for the subnormal form (bf16 only): once more from the
-  // start with the explicit conversions, one stage at a time.
+  // start, one stage at a time.
   if constexpr (Sig16<TT>::bf16) {
     if (__syncthreads_or(top >= kSubScaleLimit<TT> ? 1 : 0)) {
       clear<MB, NB>(acc);
@@ -266,10 +266,11 @@ __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         __syncthreads();
         copy_x(g.xr, smem, wave, g.xoff, s);
         load_chunk<C>(g, s, c0);
-        uint32_t o[16];
-        dequant_chunk<TT, BITS>(c0.w, TT::to_f32((uint16_t)c0.s), TT::to_f32((uint16_t)c0.b), o);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) put_piece<C>(g, 0, i, u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]});
+        const BigCst big{TT::to_f32((uint16_t)c0.s), TT::to_f32((uint16_t)c0.b)};
+        put_piece<C>(g, 0, 0, sub_group<TT, BITS, 0>(c0.w, big));
+        put_piece<C>(g, 0, 1, sub_group<TT, BITS, 1>(c0.w, big));
+        put_piece<C>(g, 0, 2, sub_group<TT, BITS, 2>(c0.w, big));
+        put_piece<C>(g, 0, 3, sub_group<TT, BITS, 3>(c0.w, big));
         stage_barrier<0>();
         last_stage<C>(g, s == last ? kv : BK, f0, acc);
       }

@@ -108,8 +108,8 @@ __device__ __forceinline__ void make_cst(const uint32_t (&sb)[C::NB], SubCst (&c
   for (int j = 0; j < C::NB; ++j) cst[j] = cst_of<typename C::TT>(sb[j] & 0xffffu, sb[j] >> 16, top);
 }
 
-template <typename C, int G>
-__device__ __forceinline__ void dequant(const TChunks<C>& c, const SubCst (&cst)[C::NB], u32x4 (&w)[C::NB]) {
+template <typename C, int G, typename K>
+__device__ __forceinline__ void dequant(const TChunks<C>& c, const K (&cst)[C::NB], u32x4 (&w)[C::NB]) {
 #pragma unroll
   for (int j = 0; j < C::NB; ++j) {
     w[j] = sub_group<typename C::TT, C::BITS, G>(c.w[j], cst[j]);
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   multiply<TT>(x1, w1, acc);
 
   // A scale too large for the subnormal form (bf16 only): once more from the
-  // start with the explicit conversions, one stage at a time.
+  // start, one stage at a time.
   if constexpr (Sig16<TT>::bf16) {
     if (__syncthreads_or(top >= kSubScaleLimit<TT> ? 1 : 0)) {
       clear<MB, NB>(acc);
@@ -329,19 +329,24 @@ __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
           clear_pieces<C::BM, C::THREADS>(smem, 4);
           __syncthreads();
         }
-        uint32_t sb[NB], o[NB][16];
+        uint32_t sb[NB];
         raw_cst<C>(g, s, sb);
+        BigCst big[NB];
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-          dequant_chunk<TT, BITS>(ca.w[j], TT::to_f32((uint16_t)(sb[j] & 0xffffu)), TT::to_f32((uint16_t)(sb[j] >> 16)),
-                                  o[j]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          get<C>(g, 0, q, x0);
-#pragma unroll
-          for (int j = 0; j < NB; ++j) w0[j] = u32x4{o[j][4 * q], o[j][4 * q + 1], o[j][4 * q + 2], o[j][4 * q + 3]};
-          multiply<TT>(x0, w0, acc);
-        }
+          big[j] = BigCst{TT::to_f32((uint16_t)(sb[j] & 0xffffu)), TT::to_f32((uint16_t)(sb[j] >> 16))};
+        get<C>(g, 0, 0, x0);
+        dequant<C, 0>(ca, big, w0);
+        multiply<TT>(x0, w0, acc);
+        get<C>(g, 0, 1, x0);
+        dequant<C, 1>(ca, big, w0);
+        multiply<TT>(x0, w0, acc);
+        get<C>(g, 0, 2, x0);
+        dequant<C, 2>(ca, big, w0);
+        multiply<TT>(x0, w0, acc);
+        get<C>(g, 0, 3, x0);
+        dequant<C, 3>(ca, big, w0);
+        multiply<TT>(x0, w0, acc);
       }
     }
   }

@@ -941,7 +941,19 @@ hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, i
     if (k <= 1024 && al16 && env_int("CPQ_QMV_DENSE", 1) != 0 && dense_small_supported(q, 1, n, k))
       return launch_dense_small(s, q, x, y, 1, n, k, true);
   }
-  if (lds > 160 * 1024) {
+  // The decode kernel for any K takes every other width, and 4/8 bits where the
+  // layouts above do not: 6-bit 2048 x 2048 5.9 -> 4.8 us, 2048 x 6144 15.8 ->
+  // 7.5; 4-bit 3520 x 3520 5.7 -> 4.8, 9984 x 3520 11.2 -> 8.7; 8-bit 3520 x
+  // 3520 6.5 -> 5.5.  Past 48 steps of 128 (a second batch per wave) or 512
+  // column blocks the shared-staging kernel is as fast at 8 bits, and past 48
+  // steps at 4-bit groups of 32 (2560 x 9984: 9.5 against 10.4).
+  if (decode_fits(q, 1, n, k, x)) {
+    const bool one_batch = k <= 6144;
+    if ((BITS != 4 && BITS != 8) || (BITS == 4 && (one_batch || q.gs > 32)) ||
+        (BITS == 8 && one_batch && (n + 15) / 16 < 512))
+      return launch_decode(s, q, x, y, 1, n, k);
+  }
+  if (lds > 160 * 1024 || (BITS != 4 && BITS != 8)) {
     // Very long rows: the small-M kernel while its slab constants fit in LDS
     // (about 500 groups per row), beyond that a prefill kernel, which keeps
     // no per-row constants in LDS.
@@ -960,9 +972,8 @@ hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, i
   } else if constexpr (BITS == 8) {
     if ((n + 15) / 16 >= 512) return launch_pf<TT, BITS, 4, 4>(s, q, x, y, n, k, lds);
     return launch_pf<TT, BITS, 8, 4>(s, q, x, y, n, k, lds);
-  } else {
-    return launch_cfg<TT, BITS, 4, 4, false>(s, q, x, y, n, k, lds);
   }
+  return hipErrorInvalidValue;
 }
 
 template <typename TT>

@@ -129,6 +129,27 @@ float small_m_us(const QuantArgs& q, const SmallPlan& sp, bool dense, int m, int
 
 }  // namespace
 
+namespace {
+
+// Up to 16 rows on the decode kernel for any K.  A workgroup holds its rows in
+// LDS: two per CU, or one where the grid is no larger than the chip.  Other
+// widths always, while staging M rows per 16 columns pays (6-bit M = 2 .. 16:
+// 3520 x 3520 9.6 .. 11.4 -> 5.8 .. 7.7 us, 1152 x 4352 13.5 .. 11.4 -> 5.6 ..
+// 7.8; 16 x 32000 x 1152 13.9 / 16.7).  4 bits: 2 x 3520 x 3520 6.8 -> 5.0, 8 x
+// 5120 x 2560 9.7 -> 6.9; short rows and, past 4 rows on few columns, K in
+// whole 256s stay (16 x 1152 x 4352 6.4 / 7.1).  8 bits: 2 x 2560 x 10048 14.5 ->
+// 11.7, 16 x 3520 x 3520 9.9 -> 7.6; many columns stay (32000 x 1152 12.4 / 13.4).
+bool decode_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
+  if (!decode_fits(q, m, n, k, x)) return false;
+  const long wgs = (n + 15) / 16;
+  if ((size_t)m * (size_t)k * 2 > 72 * 1024 && wgs > 256) return false;
+  if (q.bits != 4 && q.bits != 8) return (long)m * wgs <= 16384;
+  if (q.bits == 8) return k >= 2048 && wgs <= 400;
+  return k > 1024 && wgs < 1024 && (m <= 4 || k % 256 != 0 || wgs >= 256) && (m <= 8 || k >= 2048 || wgs >= 256);
+}
+
+}  // namespace
+
 // Y[M, N] = X[M, K] . W^T on validated operands: the kernel the shape runs
 // best on.  Up to skinny_max_m rows: at K = 4096 / 8192 / 16384 (4/8-bit, up
 // to 16 rows) the decode kernel's layout with M activation rows; else one of
@@ -165,6 +186,8 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
         sp = qmm_small_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
     }
     if (small_on && rows_on && qmv_rows_fits(q, m, n, k, x)) return launch_qmv_rows(ex.stream, q, x, y, m, n, k);
+    if (small_on && dense_env < 1 && env_int("CPQ_TILE_CFG", -1) < 0 && decode_rows(q, m, n, k, x))
+      return launch_decode(ex.stream, q, x, y, m, n, k);
     // The tiled kernel where it has a workgroup for every fourth CU at
     // least; below that (few column tiles and a K that does not split), or
     // where its K granularity does not fit, the dense form of the decode

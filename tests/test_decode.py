@@ -1,0 +1,93 @@
+"""The decode kernel for any K (up to 16 rows, every width): edges of columns,
+128-k steps, groups and waves; scales too large for the subnormal form."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from cider_press_amd import _lib
+from cider_press_amd.kernels import _ptr
+from cider_press_amd.synthetic import from_bits, make_weight, make_x, to_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(device, oracle, m, n, k, gs, bits, dtype, edit=None, skew=0):
+    rng = np.random.default_rng(m * 3 + n + k + bits)
+    w_q, s, b = make_weight(rng, n, k, gs, bits, dtype)
+    if edit:
+        edit(s, b)
+    x = make_x(rng, m, k, dtype)
+    W = device.upload(w_q.reshape(-1), "u32")
+    pad = np.zeros(skew, np.uint16)
+    S, B = (device.upload(np.concatenate([pad, t.reshape(-1)]), dtype) for t in (s, b))
+    X, Y = device.upload(x.reshape(-1), dtype), device.alloc_buffer(m * n, dtype)
+    at = lambda t: ctypes.c_void_p(t.ptr + 2 * skew)  # noqa: E731
+    cmds, L = device.commands(), _lib.lib()
+    if m == 1:
+        _lib.check(L.cpq_affine_qmv(cmds.handle, _lib.DTYPES[dtype], _ptr(W), len(W), at(S), s.size, at(B), b.size,
+                                    _ptr(X), X.alloc_len, _ptr(Y), len(Y), k, gs, bits))
+    else:
+        _lib.check(L.cpq_affine_qmm_t(cmds.handle, _lib.DTYPES[dtype], _ptr(W), len(W), at(S), s.size, at(B), b.size,
+                                      _ptr(X), len(X), _ptr(Y), len(Y), m, n, k, gs, bits))
+    cmds.commit_and_wait()
+    w = from_bits(oracle.dequantize(w_q, s, b, n, k, gs, bits, dtype), dtype).astype(np.float64)
+    return (from_bits(Y.to_numpy().reshape(m, n), dtype).astype(np.float64),
+            from_bits(x, dtype).astype(np.float64) @ w.T, dtype)
+
+
+def _close(y, ref, dtype):
+    """Rounding the output to T moves each value by at most T's unit roundoff
+    (2^-8 with bf16's 8 significant bits, 2^-11 with f16's 11); fp32 sums of K
+    terms add a few 2^-24 of the terms' magnitude, here under 1e-5 of the norm."""
+    assert np.isfinite(y).all()
+    bound = (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) + 1e-5
+    assert np.linalg.norm(y - ref) <= bound * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("waves", [1, 3, 12])
+@pytest.mark.parametrize("m,n,k,gs,bits,dtype,skew", [
+    (1, 1, 32, 32, 6, "bf16", 0),        # one column, a quarter step
+    (1, 17, 96, 32, 3, "f16", 1),        # one column past a block, tables on an odd element
+    (1, 131, 2080, 32, 5, "bf16", 1),    # 65 groups a row
+    (1, 48, 4416, 64, 2, "f16", 0),      # 69 groups, half a step at the end, several batches a wave
+    (1, 40, 1152, 64, 4, "bf16", 1),
+    (1, 33, 1152, 128, 8, "f16", 0),
+    (2, 64, 3520, 64, 4, "bf16", 1),
+    (5, 96, 2112, 64, 8, "f16", 1),
+    (16, 160, 1376, 32, 6, "bf16", 0),
+    (13, 96, 896, 128, 3, "bf16", 0),
+])
+def test_decode(device, oracle, monkeypatch, waves, m, n, k, gs, bits, dtype, skew):
+    monkeypatch.setenv("CPQ_DECODE_WAVES", str(waves))
+    _close(*_run(device, oracle, m, n, k, gs, bits, dtype, skew=skew))
+
+
+@pytest.mark.parametrize("m", [1, 3])
+def test_decode_large_scales(device, oracle, m):
+    """bf16 scales of 2^104 and above overflow the subnormal form."""
+    def edit(s, b):
+        for col, value in ((5, 2.0 ** 104), (40, 2.0 ** 112)):
+            s[col, 2] = to_bits(np.float32([value]), "bf16")[0]
+            b[col, 2] = to_bits(np.float32([-2.0 ** 100]), "bf16")[0]
+
+    y, ref, dtype = _run(device, oracle, m, 64, 1280, 64, 6, "bf16", edit)
+    for cols in ([5], [40], [c for c in range(64) if c not in (5, 40)]):
+        _close(y[:, cols], ref[:, cols], dtype)
+
+
+def test_decode_skips_values_past_k(device, oracle):
+    """Rows of X follow one another: an infinity at the next row's start must not
+    reach the partial last step of the row before it."""
+    m, n, k, gs, bits = 3, 32, 1184, 32, 6
+    rng = np.random.default_rng(2)
+    w_q, s, b = make_weight(rng, n, k, gs, bits, "bf16")
+    x = make_x(rng, m, k, "bf16")
+    x[1, 0] = 0x7F80
+    W, S, B = (device.upload(t.reshape(-1), d) for t, d in ((w_q, "u32"), (s, "bf16"), (b, "bf16")))
+    X, Y, cmds = device.upload(x.reshape(-1), "bf16"), device.alloc_buffer(m * n, "bf16"), device.commands()
+    _lib.check(_lib.lib().cpq_affine_qmm_t(cmds.handle, _lib.DTYPES["bf16"], _ptr(W), len(W), _ptr(S), len(S), _ptr(B),
+                                           len(B), _ptr(X), len(X), _ptr(Y), len(Y), m, n, k, gs, bits))
+    cmds.commit_and_wait()
+    y = from_bits(Y.to_numpy().reshape(m, n), "bf16")
+    assert np.isfinite(y[[0, 2]]).all() and not np.isfinite(y[1]).any()
