@@ -129,6 +129,11 @@ hipError_t launch_qvm(hipStream_t s, const QvmPlan& p, void* scratch, const Quan
 size_t moe_sort_scratch_bytes(int rows, int n_experts);
 hipError_t launch_moe_route(hipStream_t s, int logits_dtype, const void* logits, int tokens, int n_experts, int top_k,
                             int normalize, uint32_t* experts, float* scores);
+// Both in one launch, for a few tokens.
+bool moe_route_sort_fits(int tokens);
+hipError_t launch_moe_route_sort(hipStream_t s, int logits_dtype, const void* logits, int tokens, int n_experts,
+                                 int top_k, int normalize, uint32_t* experts, float* scores, uint32_t* lhs,
+                                 uint32_t* rhs, uint32_t* inv, uint32_t* offsets);
 hipError_t launch_moe_sort(hipStream_t s, const uint32_t* experts, int rows, int top_k, int n_experts,
                            uint32_t* scratch, uint32_t* lhs, uint32_t* rhs, uint32_t* inv, uint32_t* offsets);
 hipError_t launch_moe_combine(hipStream_t s, int dtype, const void* y, const float* scores, const uint32_t* inv,

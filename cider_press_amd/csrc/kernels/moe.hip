@@ -50,15 +50,12 @@ __device__ __forceinline__ unsigned long long rank_key(float p, int e) {
   return ((unsigned long long)__float_as_uint(p) << 32) | (uint32_t)~(uint32_t)e;
 }
 
-// One wave per token.  Lane l holds experts l + 64 i, i < NV (NV = ceil(E/64)).
+// One token by one wave.  Lane l holds experts l + 64 i, i < NV (NV = ceil(E/64));
+// lane j < top_k returns pick j and its (normalized) score.
 template <int L, int NV>
-__global__ __launch_bounds__(256) void route_kernel(const void* __restrict__ logits, int tokens, int n_experts,
-                                                    int top_k, int normalize, uint32_t* __restrict__ experts,
-                                                    float* __restrict__ scores) {
+__device__ __forceinline__ void route_token(const void* logits, size_t row, int n_experts, int top_k, int normalize,
+                                            int& pick, float& score) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= tokens) return;  // whole waves leave together
-  const size_t row = (size_t)t * n_experts;
   float v[NV];
   bool live[NV];
   float m = -INFINITY;
@@ -107,9 +104,106 @@ __global__ __launch_bounds__(256) void route_kernel(const void* __restrict__ log
   // The picks' sum in pick order (lane 0 .. k-1), the order a serial loop uses.
   float psum = 0.f;
   for (int j = 0; j < top_k; ++j) psum += __shfl(my_p, j, 64);
+  pick = my_e;
+  score = normalize ? my_p / psum : my_p;
+}
+
+// One wave per token.
+template <int L, int NV>
+__global__ __launch_bounds__(256) void route_kernel(const void* __restrict__ logits, int tokens, int n_experts,
+                                                    int top_k, int normalize, uint32_t* __restrict__ experts,
+                                                    float* __restrict__ scores) {
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= tokens) return;  // whole waves leave together
+  int pick;
+  float score;
+  route_token<L, NV>(logits, (size_t)t * n_experts, n_experts, top_k, normalize, pick, score);
   if (lane < top_k) {
-    experts[(size_t)t * top_k + lane] = (uint32_t)my_e;
-    scores[(size_t)t * top_k + lane] = normalize ? my_p / psum : my_p;
+    experts[(size_t)t * top_k + lane] = (uint32_t)pick;
+    scores[(size_t)t * top_k + lane] = score;
+  }
+}
+
+// Rank of a lane among the earlier lanes of its wave with the same value, and
+// how many lanes have it (64 lane reads, no LDS round trips).
+__device__ __forceinline__ void lane_rank(uint32_t e, uint32_t& rank, uint32_t& same) {
+  const int lane = threadIdx.x & 63;
+  rank = same = 0;
+#pragma unroll 8
+  for (int i = 0; i < 64; ++i) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)e, i);
+    const uint32_t eq = (o == e) ? 1u : 0u;
+    same += eq;
+    rank += (i < lane) ? eq : 0u;
+  }
+}
+
+// Routing and sort of a few tokens (at most kFusedTokens, so at most 512 rows)
+// by one workgroup in one launch: decode steps otherwise spend four launches
+// and their gaps on a few hundred bytes.  16 waves route a token each at a
+// time into LDS; then wave w ranks rows 64w .. 64w + 63, thread e adds the waves'
+// counts of expert e, a scan over the experts gives the starts, and each row's
+// position is its expert's start, the earlier waves' counts and its rank.
+constexpr int kFusedTokens = 32;
+template <int L, int NV>
+__global__ __launch_bounds__(1024) void route_sort_kernel(const void* __restrict__ logits, int tokens, int n_experts,
+                                                          int top_k, int normalize, uint32_t* __restrict__ experts,
+                                                          float* __restrict__ scores, uint32_t* __restrict__ lhs,
+                                                          uint32_t* __restrict__ rhs, uint32_t* __restrict__ inv,
+                                                          uint32_t* __restrict__ offsets) {
+  constexpr int ROWS = kFusedTokens * kMaxTopK, RW = ROWS / 64;
+  __shared__ uint32_t pick_of[ROWS];
+  __shared__ uint32_t start[kMaxExperts];
+  __shared__ uint32_t wave_total[16];
+  __shared__ uint8_t cnt[RW][kMaxExperts];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rows = tokens * top_k;
+  for (int i = tid; i < RW * kMaxExperts / 4; i += 1024) reinterpret_cast<uint32_t*>(&cnt[0][0])[i] = 0u;
+  for (int t = wave; t < tokens; t += 16) {
+    int pick;
+    float score;
+    route_token<L, NV>(logits, (size_t)t * n_experts, n_experts, top_k, normalize, pick, score);
+    if (lane < top_k) {
+      const int r = t * top_k + lane;
+      pick_of[r] = (uint32_t)pick;
+      experts[r] = (uint32_t)pick;
+      scores[r] = score;
+    }
+  }
+  __syncthreads();  // picks in LDS, cnt cleared
+  const bool live = tid < rows;
+  const uint32_t e = live ? pick_of[tid] : 0xffffffffu;
+  uint32_t rank = 0, same = 0;
+  if (wave * 64 < rows) {
+    lane_rank(e, rank, same);
+    if (live && rank + 1 == same) cnt[wave][e] = (uint8_t)same;
+  }
+  __syncthreads();
+  // Exclusive scan of the experts' totals: inside a wave, then over the waves.
+  uint32_t total = 0;
+#pragma unroll
+  for (int w = 0; w < RW; ++w) total += cnt[w][tid];
+  uint32_t upto = total;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t o = __shfl_up(upto, d, 64);
+    upto += lane >= d ? o : 0u;
+  }
+  if (lane == 63) wave_total[wave] = upto;
+  __syncthreads();
+  uint32_t before = 0;
+  for (int w = 0; w < wave; ++w) before += wave_total[w];
+  start[tid] = before + upto - total;
+  if (tid < n_experts) offsets[tid] = before + upto - total;
+  if (tid == 0) offsets[n_experts] = (uint32_t)rows;
+  __syncthreads();
+  if (live) {
+    uint32_t pos = start[e] + rank;
+    for (int w = 0; w < wave; ++w) pos += cnt[w][e];
+    lhs[pos] = (uint32_t)(tid / top_k);
+    rhs[pos] = e;
+    inv[tid] = pos;
   }
 }
 
@@ -160,9 +254,7 @@ __global__ __launch_bounds__(1024) void sort_scan_kernel(uint32_t* __restrict__ 
 }
 
 // Four waves per block of kSortRows rows, wave w on rows 64w .. 64w+63 of
-// the block.  A lane's rank among the earlier lanes of its wave with the same
-// expert comes from 64 lane reads (no LDS round trips); the last lane of each
-// (wave, expert) run publishes the run's length, and a lane's sorted position
+// the block; the last lane of each (wave, expert) run publishes the run's length, and a lane's sorted position
 // is its block's start for the expert, plus the counts of the earlier waves,
 // plus its rank -- so equal experts keep row order.
 __global__ __launch_bounds__(256) void sort_scatter_kernel(const uint32_t* __restrict__ experts, int rows, int top_k,
@@ -170,19 +262,13 @@ __global__ __launch_bounds__(256) void sort_scatter_kernel(const uint32_t* __res
                                                            uint32_t* __restrict__ lhs, uint32_t* __restrict__ rhs,
                                                            uint32_t* __restrict__ inv) {
   __shared__ uint32_t cnt[4][kMaxExperts];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6;
   for (int i = threadIdx.x; i < 4 * kMaxExperts; i += 256) (&cnt[0][0])[i] = 0u;
   const int r = blockIdx.x * kSortRows + threadIdx.x;
   const bool live = r < rows;
   const uint32_t e = live ? experts[r] : 0xffffffffu;
-  uint32_t rank = 0, same = 0;
-#pragma unroll 8
-  for (int i = 0; i < 64; ++i) {
-    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)e, i);
-    const uint32_t eq = (o == e) ? 1u : 0u;
-    same += eq;
-    rank += (i < lane) ? eq : 0u;
-  }
+  uint32_t rank, same;
+  lane_rank(e, rank, same);
   __syncthreads();  // cnt cleared
   if (live && rank + 1 == same) cnt[wave][e] = same;
   __syncthreads();
@@ -253,6 +339,39 @@ hipError_t launch_route_nv(hipStream_t s, const void* logits, int tokens, int n_
   else CPQ_ROUTE(16);
 #undef CPQ_ROUTE
   return hipGetLastError();
+}
+
+template <int L>
+hipError_t launch_route_sort_nv(hipStream_t s, const void* logits, int tokens, int n_experts, int top_k, int normalize,
+                                uint32_t* experts, float* scores, uint32_t* lhs, uint32_t* rhs, uint32_t* inv,
+                                uint32_t* offsets) {
+  const int nv = (n_experts + 63) / 64;
+#define CPQ_ROUTE(NVV)                                                                                               \
+  hipLaunchKernelGGL((route_sort_kernel<L, NVV>), dim3(1), dim3(1024), 0, s, logits, tokens, n_experts, top_k, normalize, \
+                     experts, scores, lhs, rhs, inv, offsets)
+  if (nv <= 1) CPQ_ROUTE(1);
+  else if (nv <= 2) CPQ_ROUTE(2);
+  else if (nv <= 4) CPQ_ROUTE(4);
+  else if (nv <= 8) CPQ_ROUTE(8);
+  else CPQ_ROUTE(16);
+#undef CPQ_ROUTE
+  return hipGetLastError();
+}
+
+bool moe_route_sort_fits(int tokens) { return tokens >= 1 && tokens <= kFusedTokens; }
+
+hipError_t launch_moe_route_sort(hipStream_t s, int logits_dtype, const void* logits, int tokens, int n_experts,
+                                 int top_k, int normalize, uint32_t* experts, float* scores, uint32_t* lhs,
+                                 uint32_t* rhs, uint32_t* inv, uint32_t* offsets) {
+  if (!moe_route_sort_fits(tokens)) return hipErrorInvalidValue;
+  if (logits_dtype == CPQ_DTYPE_F32)
+    return launch_route_sort_nv<0>(s, logits, tokens, n_experts, top_k, normalize, experts, scores, lhs, rhs, inv,
+                                   offsets);
+  if (logits_dtype == CPQ_DTYPE_F16)
+    return launch_route_sort_nv<1>(s, logits, tokens, n_experts, top_k, normalize, experts, scores, lhs, rhs, inv,
+                                   offsets);
+  return launch_route_sort_nv<2>(s, logits, tokens, n_experts, top_k, normalize, experts, scores, lhs, rhs, inv,
+                                 offsets);
 }
 
 hipError_t launch_moe_route(hipStream_t s, int logits_dtype, const void* logits, int tokens, int n_experts, int top_k,

@@ -822,6 +822,11 @@ cpq_status cpq_moe_route(cpq_commands* cmds, cpq_dtype logits_dtype, const void*
                                               " bytes of session scratch; the session holds " +
                                               std::to_string(cmds->scratch_bytes) +
                                               " (CPQ_SESSION_SCRATCH_MB sets it when the session is made)");
+  if (cpq::moe_route_sort_fits((int)tokens))
+    return cpq::launched(cpq::launch_moe_route_sort(cmds->stream, (int)logits_dtype, logits, (int)tokens,
+                                                    (int)n_experts, (int)top_k, normalize, experts, scores, lhs, rhs,
+                                                    inv, offsets),
+                         "moe_route launch");
   // The scratch head holds the prefill kernel's arrival counters; the sort's
   // block histograms go after it.
   uint32_t* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + cpq::kWideCounterBytes);

@@ -189,3 +189,21 @@ def test_moe_projection_end_to_end(device, library, oracle):
     ref = np.einsum("tk,tkn->tn", sc, dense_t)
     rep = oracle.tolerance_report(O.to_numpy()[: tokens * n].reshape(tokens, n), ref, x, kd, "bf16")
     assert rep["ok"], rep
+
+
+@pytest.mark.parametrize("tokens,E,k,normalize,dtype", [
+    (4, 128, 8, True, "bf16"),     # one wave of rows
+    (32, 1000, 16, True, "f32"),   # the most tokens and rows of the one-launch form
+    (31, 4, 4, False, "f16"),      # every row of a token on the 4 experts: long equal runs
+    (17, 65, 5, True, "bf16"),     # a second token for one wave, rows end inside a wave
+])
+def test_route_and_sort_few_tokens(device, tokens, E, k, normalize, dtype):
+    rng = np.random.default_rng(tokens * 11 + E + k)
+    bits, lg = _logits(rng, tokens, E, dtype)
+    got, _, _ = run_route(device, bits, dtype, tokens, E, k, normalize)
+    ex, sc = np_route(lg, k, normalize)
+    assert np.array_equal(got["experts"].reshape(tokens, k), ex)
+    np.testing.assert_allclose(got["scores"].reshape(tokens, k), sc, rtol=2e-6, atol=1e-7)
+    lhs, rhs, inv, offsets = np_sort(got["experts"], k, E)
+    assert np.array_equal(got["lhs"], lhs) and np.array_equal(got["rhs"], rhs)
+    assert np.array_equal(got["inv"], inv) and np.array_equal(got["offsets"], offsets)
