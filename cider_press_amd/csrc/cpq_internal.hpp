@@ -315,8 +315,26 @@ hipError_t launch_stream_read(hipStream_t s, const void* const* regions, const s
                               uint32_t* sink, int n_wg, int variant);
 int stream_read_variant_count();
 
-// Integer from the environment (tuning and test hooks), dflt when unset.
+// Integer from the environment (tuning and test hooks), dflt when unset.  An op
+// looks up about ten of them; inside a HookScope they cost one look over the
+// environment for any CPQ_ name.
+struct HookScope {
+  HookScope() : outer(state) {
+    if (state == kOutside) state = any() ? kSome : kNone;
+  }
+  ~HookScope() { state = outer; }
+  HookScope(const HookScope&) = delete;
+  HookScope& operator=(const HookScope&) = delete;
+  enum State { kOutside, kNone, kSome };
+  static thread_local State state;
+
+ private:
+  static bool any();
+  State outer;
+};
+
 inline int env_int(const char* name, int dflt) {
+  if (HookScope::state == HookScope::kNone) return dflt;
   const char* e = std::getenv(name);
   return e && *e ? std::atoi(e) : dflt;
 }

@@ -227,8 +227,10 @@ namespace {
 
 cpq_status route_matmul(cpq_commands* cmds, const QuantArgs& q, const void* x, void* y, int m, int n, int k,
                         const char* op) {
-  const std::string what = std::string(op) + (m <= skinny_max_m(q, n, k) ? " (small-M) launch" : " (prefill) launch");
-  return launched(launch_matmul(session_ctx(cmds), q, x, y, m, n, k), what.c_str());
+  const HookScope hooks;
+  const hipError_t e = launch_matmul(session_ctx(cmds), q, x, y, m, n, k);
+  if (e == hipSuccess) return CPQ_OK;
+  return hip_fail(e, (std::string(op) + (m <= skinny_max_m(q, n, k) ? " (small-M) launch" : " (prefill) launch")).c_str());
 }
 
 }  // namespace
@@ -508,6 +510,7 @@ cpq_status cpq_affine_qmv(cpq_commands* cmds, cpq_dtype dtype, const uint32_t* w
   st = cpq::check_ptrs("affine_qmv", w_q, scales, biases, x, y);
   if (st != CPQ_OK) return st;
   cpq::QuantArgs q{w_q, scales, biases, (int)group_size, (int)bits, dtype};
+  const cpq::HookScope hooks;
   return cpq::launched(cpq::launch_qmv(cmds->stream, q, x, y, (int)y_len, (int)in_vec_size),
                        "affine_qmv launch");
 }
@@ -758,6 +761,7 @@ cpq_status cpq_affine_qmm_n(cpq_commands* cmds, cpq_dtype dtype, const uint32_t*
                        k ? biases : y, k ? x : y, y);
   if (st != CPQ_OK) return st;
   cpq::QuantArgs q{w_q, scales, biases, (int)group_size, (int)bits, dtype};
+  const cpq::HookScope hooks;
   if (m == 1 && k > 0 && (reinterpret_cast<uintptr_t>(x) & 3u) == 0 && cpq::qvm_fits(q, (int)n, (int)k)) {
     // Decode (qvm): the VALU kernel, K split over parts that meet in the
     // session scratch when it holds them (the plan depends on the session's

@@ -19,7 +19,17 @@ thread_local std::string g_last_error;
 constexpr size_t kAllocGranule = 512;  // device.rs:191-224 rounds every allocation to 512 B
 }  // namespace
 
+extern char** environ;
+
 namespace cpq {
+
+thread_local HookScope::State HookScope::state = HookScope::kOutside;
+
+bool HookScope::any() {
+  for (char** e = environ; e && *e; ++e)
+    if (std::strncmp(*e, "CPQ_", 4) == 0) return true;
+  return false;
+}
 
 cpq_status fail(cpq_status st, const std::string& msg) {
   g_last_error = msg;

@@ -310,8 +310,9 @@ class KernelLibrary:
         return bool(_lib.lib().cpq_kernel_available(_lib.DTYPES[dtype], group_size, bits))
 
 
-def _ptr(buf) -> ctypes.c_void_p:
-    return ctypes.c_void_p(None if buf is None else buf.ptr)
+def _ptr(buf):
+    """Device address for a void* argument (an int: no ctypes object per call)."""
+    return None if buf is None else buf.ptr
 
 
 from . import dequantize, embed, gather, moe, qmm, qmv  # noqa: E402,F401
