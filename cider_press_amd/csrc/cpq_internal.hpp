@@ -152,6 +152,10 @@ hipError_t launch_qmv(hipStream_t s, const QuantArgs& q, const void* x, void* y,
 // aligned.
 bool decode_fits(const QuantArgs& q, int m, int n, int k, const void* x);
 hipError_t launch_decode(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
+// The same where a workgroup's rows do not fit its LDS at once: each wave stages
+// its activations in phases.
+bool decode_phased_fits(const QuantArgs& q, int m, int n, int k, const void* x);
+hipError_t launch_decode_phased(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
 
 // A batch folded into a grid dimension (MLX's adjust_matrix_offsets):
 // element z (row-major over shape[0..nd)) takes its operands at

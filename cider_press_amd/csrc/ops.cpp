@@ -150,6 +150,24 @@ bool decode_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
 
 }  // namespace
 
+namespace {
+
+// Rows that exceed a workgroup's LDS, staged in phases.  Up to 12 rows every
+// wave still has whole batches in LDS, up to K = 12288 in two phases; the grid
+// has to give half the CUs a workgroup and no CU two.  8 x 4096 x 12288 8-bit
+// 24.2 -> 20.0 us, 8 x 3520 x 9984 6-bit 19.8 -> 16.5 and 3-bit 19.1 -> 14.9, 12 x
+// 2048 x 7936 8-bit 16.9 -> 16.2, 8 x 2560 x 10048 4-bit 18.3 -> 13.7.  Others
+// stay: 16 rows (16 x 3520 x 9984 6-bit 20.0 / 22.2), K = 16128 (12 x 2048 6-bit
+// 22.3 / 23.5), 4 bits in whole 256s of K (10 x 3072 x 8448 10.1 / 13.7), 72
+// workgroups (8 x 1152 x 16384 20.7 / 22.8), 768 (8 x 12288 x 4096 19.6 / 24.2).
+bool decode_phased_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
+  const long wgs = (n + 15) / 16;
+  if (m > 12 || k > 12288 || wgs < 128 || wgs > 256 || (q.bits == 4 && k % 256 == 0)) return false;
+  return !decode_fits(q, m, n, k, x) && decode_phased_fits(q, m, n, k, x);
+}
+
+}  // namespace
+
 // Y[M, N] = X[M, K] . W^T on validated operands: the kernel the shape runs
 // best on.  Up to skinny_max_m rows: at K = 4096 / 8192 / 16384 (4/8-bit, up
 // to 16 rows) the decode kernel's layout with M activation rows; else one of
@@ -185,9 +203,13 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
       if (sp.split > 0 && sp.scratch_bytes > ex.scratch_bytes)
         sp = qmm_small_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
     }
+    const int phased = env_int("CPQ_DECODE_PHASED", -1);  // 1 where it applies, 0 off (test hook)
+    if (phased == 1 && decode_phased_fits(q, m, n, k, x)) return launch_decode_phased(ex.stream, q, x, y, m, n, k);
     if (small_on && rows_on && qmv_rows_fits(q, m, n, k, x)) return launch_qmv_rows(ex.stream, q, x, y, m, n, k);
     if (small_on && dense_env < 1 && env_int("CPQ_TILE_CFG", -1) < 0 && decode_rows(q, m, n, k, x))
       return launch_decode(ex.stream, q, x, y, m, n, k);
+    if (small_on && dense_env < 1 && phased != 0 && env_int("CPQ_TILE_CFG", -1) < 0 && decode_phased_rows(q, m, n, k, x))
+      return launch_decode_phased(ex.stream, q, x, y, m, n, k);
     // The tiled kernel where it has a workgroup for every fourth CU at
     // least; below that (few column tiles and a K that does not split), or
     // where its K granularity does not fit, the dense form of the decode

@@ -91,3 +91,25 @@ def test_decode_skips_values_past_k(device, oracle):
     cmds.commit_and_wait()
     y = from_bits(Y.to_numpy().reshape(m, n), "bf16")
     assert np.isfinite(y[[0, 2]]).all() and not np.isfinite(y[1]).any()
+
+
+@pytest.mark.parametrize("m,n,k,gs,bits,dtype,skew", [
+    (16, 32, 128, 64, 6, "bf16", 0),      # one step, one wave
+    (13, 64, 6496, 32, 3, "f16", 1),      # a partial last step, odd group counts
+    (7, 64, 12288, 64, 8, "bf16", 0),     # two phases, whole
+    (16, 96, 9632, 32, 5, "bf16", 1),     # 9 waves, a last phase of part of a batch, a last wave with fewer steps
+    (12, 2080, 8064, 128, 8, "f16", 0),   # as the route takes it
+    (2, 32, 40960, 64, 4, "f16", 1),      # one row block, many batches a phase
+    (16, 32, 30720, 64, 2, "bf16", 0),    # many phases
+])
+def test_decode_phased(device, oracle, monkeypatch, m, n, k, gs, bits, dtype, skew):
+    """Activations staged in phases, where the rows exceed a workgroup's LDS."""
+    monkeypatch.setenv("CPQ_DECODE_PHASED", "1")
+
+    def edit(s, b):
+        if dtype == "bf16":  # a wave that meets a large scale goes over its phases again
+            s[5, -1], b[5, -1] = to_bits(np.float32([2.0 ** 104, -2.0 ** 100]), "bf16")
+
+    y, ref, dtype = _run(device, oracle, m, n, k, gs, bits, dtype, edit, skew)
+    for cols in ([5], [c for c in range(n) if c != 5]):
+        _close(y[:, cols], ref[:, cols], dtype)
