@@ -390,6 +390,16 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wave's LDS accesses around this point: lanes of one wave that read
+// each other's LDS writes (or overwrite what others were reading) need it on
+// both sides of the writes.  No instruction: the LDS keeps a wave's order, this
+// keeps the compiler's.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Wave64 sum via DPP-friendly butterfly.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -214,9 +214,11 @@ __global__ __launch_bounds__(64 * MAXW) void decode_kernel(const uint32_t* __res
         *reinterpret_cast<u32x4*>(xw + ((size_t)r * hold + (p >> 4)) * (STEP * 2) + (((p & 15) ^ swz_key(r)) << 4)) = v;
     };
     // The phase of steps t0 .. t0 + hold - 1 takes the place of the one before
-    // (the wave's own LDS: its reads of that are behind it).
+    // (the wave's own LDS, no barrier: other lanes read what this one writes, so
+    // the phases' reads and writes are kept in order within the wave).
     auto next_phase = [&](int t0) {
       const int held = min(hold, nt - t0) * 16;
+      wave_lds_order();
       for (int r0 = 0; r0 < m; r0 += 4)
         for (int p = lane; p < held; p += 64) {
           const int kk = (u0 + t0) * STEP + p * 8;
@@ -233,6 +235,7 @@ __global__ __launch_bounds__(64 * MAXW) void decode_kernel(const uint32_t* __res
               *reinterpret_cast<u32x4*>(xw + ((size_t)(r0 + r) * hold + (p >> 4)) * (STEP * 2) +
                                         (((p & 15) ^ swz_key(r0 + r)) << 4)) = v[r];
         }
+      wave_lds_order();
       q.xrow -= hold * (STEP * 2);
     };
     Batch<BITS, GS_SHIFT> b0, b1;
@@ -259,6 +262,7 @@ __global__ __launch_bounds__(64 * MAXW) void decode_kernel(const uint32_t* __res
         for (int r = 0; r < 4; ++r)
           if (r0 + r < m) xput(r0 + r, p0 + lane, v[r]);
       }
+    wave_lds_order();  // lanes read what other lanes staged
     for (int t0 = 0; t0 < nt; t0 += 2 * BATCH) {
       if (PHASED && t0 && t0 % hold == 0) next_phase(t0);
       if (t0 + BATCH < nt) load_batch<BITS, GS_SHIFT>(q, t0 + BATCH, b1);

@@ -113,3 +113,31 @@ def test_decode_phased(device, oracle, monkeypatch, m, n, k, gs, bits, dtype, sk
     y, ref, dtype = _run(device, oracle, m, n, k, gs, bits, dtype, edit, skew)
     for cols in ([5], [c for c in range(n) if c != 5]):
         _close(y[:, cols], ref[:, cols], dtype)
+
+
+@pytest.mark.parametrize("m,n,k,gs,bits,phased,large", [
+    (1, 64, 6112, 32, 6, False, False),
+    (16, 64, 2080, 32, 5, False, True),   # rows staged four at a time, the large-scale pass reads them again
+    (16, 64, 9632, 32, 3, True, False),   # a wave's lanes refill what other lanes were reading
+    (7, 64, 12288, 64, 8, True, True),
+])
+def test_decode_lanes_read_what_others_staged(device, oracle, monkeypatch, m, n, k, gs, bits, phased, large):
+    """Lanes of a wave read activations that other lanes wrote to LDS.  Calls on
+    other values in between leave theirs there: whoever read early would see
+    them, so every call gives the first one's bits."""
+    if phased:
+        monkeypatch.setenv("CPQ_DECODE_PHASED", "1")
+
+    def edit(s, b):
+        if large:
+            s[5, -1], b[5, -1] = to_bits(np.float32([2.0 ** 104, -2.0 ** 100]), "bf16")
+
+    def other(s, b):
+        s[:] = to_bits(np.full(s.size, 0.5, np.float32), "bf16").reshape(s.shape)
+
+    y, ref, dtype = _run(device, oracle, m, n, k, gs, bits, "bf16", edit)
+    for cols in ([5], [c for c in range(n) if c != 5]):
+        _close(y[:, cols], ref[:, cols], dtype)
+    for _ in range(3):
+        _run(device, oracle, m, n, k, gs, bits, "bf16", other)
+        assert np.array_equal(_run(device, oracle, m, n, k, gs, bits, "bf16", edit)[0], y)
