@@ -148,8 +148,8 @@ hipError_t launch_embed(hipStream_t s, const QuantArgs& q, const uint32_t* ids, 
 hipError_t launch_qmv(hipStream_t s, const QuantArgs& q, const void* x, void* y, int n, int k);
 
 // The decode kernel for up to 16 rows at every width (kernels/decode.hip): K a
-// multiple of 32, M * K * 2 bytes and the K parts within LDS, x and w 16-byte
-// aligned.
+// multiple of 32 up to 2^25, M * K * 2 bytes and the K parts within LDS, x and w
+// 16-byte aligned.
 bool decode_fits(const QuantArgs& q, int m, int n, int k, const void* x);
 hipError_t launch_decode(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
 // The same where a workgroup's rows do not fit its LDS at once: each wave stages

@@ -374,7 +374,8 @@ hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, i
 namespace {
 
 bool decode_takes(const QuantArgs& q, int m, int n, int k, const void* x) {
-  if (m < 1 || m > 16 || n < 1 || k < 32 || k % 32 != 0 || k > (1 << 21)) return false;
+  // 16 rows of X and of W within the 32-bit ranges of their buffers.
+  if (m < 1 || m > 16 || n < 1 || k < 32 || k % 32 != 0 || k > (1 << 25)) return false;
   if (q.gs != 32 && q.gs != 64 && q.gs != 128) return false;
   return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(q.w)) & 15u) == 0;
 }

@@ -752,6 +752,10 @@ int shift_of(int gs) {
   return s;
 }
 
+// Dynamic LDS the shared-staging kernel can be given (its static LDS and the
+// rest of 160 KiB left over).
+constexpr size_t kSharedLds = 160 * 1024 - 1024;
+
 template <typename TT, int BITS, int WAVES, int PF, bool EXACT>
 hipError_t launch_cfg(hipStream_t s, const QuantArgs& q, const void* x, void* y, int n, int k,
                       size_t lds) {
@@ -768,7 +772,7 @@ hipError_t launch_cfg(hipStream_t s, const QuantArgs& q, const void* x, void* y,
                                  (int)(160 * 1024 - fa.sharedSizeBytes));
     }();
     if (attr != hipSuccess) return attr;
-    if (lds > 160 * 1024 - 1024) return hipErrorInvalidValue;
+    if (lds > kSharedLds) return hipErrorInvalidValue;
   }
   hipLaunchKernelGGL((qmv_kernel<TT, BITS, WAVES, PF, EXACT>), dim3((unsigned)((n + 15) / 16)),
                      dim3(64 * WAVES), lds, s, q.w, static_cast<const uint16_t*>(q.scales),
@@ -941,23 +945,26 @@ hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, i
     if (k <= 1024 && al16 && env_int("CPQ_QMV_DENSE", 1) != 0 && dense_small_supported(q, 1, n, k))
       return launch_dense_small(s, q, x, y, 1, n, k, true);
   }
+  // The shared-staging kernel keeps x and 16 rows' constants in LDS: 4/8 bits, K up
+  // to about 16200 at groups of 32.
+  const bool shared = (BITS == 4 || BITS == 8) && lds <= kSharedLds;
   // The decode kernel for any K takes every other width, and 4/8 bits where the
   // layouts above do not: 6-bit 2048 x 2048 5.9 -> 4.8 us, 2048 x 6144 15.8 ->
   // 7.5; 4-bit 3520 x 3520 5.7 -> 4.8, 9984 x 3520 11.2 -> 8.7; 8-bit 3520 x
   // 3520 6.5 -> 5.5.  Past 48 steps of 128 (a second batch per wave) or 512
-  // column blocks the shared-staging kernel is as fast at 8 bits, and past 48
-  // steps at 4-bit groups of 32 (2560 x 9984: 9.5 against 10.4).
-  if (decode_fits(q, 1, n, k, x)) {
-    const bool one_batch = k <= 6144;
-    if ((BITS != 4 && BITS != 8) || (BITS == 4 && (one_batch || q.gs > 32)) ||
-        (BITS == 8 && one_batch && (n + 15) / 16 < 512))
-      return launch_decode(s, q, x, y, 1, n, k);
-  }
-  if (lds > 160 * 1024 || (BITS != 4 && BITS != 8)) {
-    // Very long rows: the small-M kernel while its slab constants fit in LDS
-    // (about 500 groups per row), beyond that a prefill kernel, which keeps
-    // no per-row constants in LDS.
-    if (skinny_fits(k, q.gs)) return launch_qmm_skinny(s, q, x, y, 1, n, k);
+  // column blocks the shared-staging kernel, where it fits, is as fast at 8 bits,
+  // and past 48 steps at 4-bit groups of 32 (2560 x 9984: 9.5 against 10.4).
+  // Where it does not fit, a prefill kernel on one row took 219 us against 29.5 at
+  // 4-bit 5120 x 17920, groups of 32.
+  const bool one_batch = k <= 6144;
+  if (decode_fits(q, 1, n, k, x) &&
+      (!shared || (BITS == 4 && (one_batch || q.gs > 32)) || (BITS == 8 && one_batch && (n + 15) / 16 < 512)))
+    return launch_decode(s, q, x, y, 1, n, k);
+  if (!shared) {
+    // Rows past what either holds in LDS (K of about 75000): the decode kernel
+    // with x in phases (4-bit 512 x 81920 53 us, 864 on a prefill kernel); beyond
+    // its 32-bit ranges a prefill kernel.
+    if (decode_phased_fits(q, 1, n, k, x)) return launch_decode_phased(s, q, x, y, 1, n, k);
     return launch_qmm_unsplit(s, q, x, y, 1, n, k);
   }
   const int units = k / 128;

@@ -63,6 +63,24 @@ def test_decode(device, oracle, monkeypatch, waves, m, n, k, gs, bits, dtype, sk
     _close(*_run(device, oracle, m, n, k, gs, bits, dtype, skew=skew))
 
 
+@pytest.mark.parametrize("n,k,gs,bits,dtype", [
+    (48, 16224, 32, 4, "bf16"),      # x and 16 rows' constants: 159 to 160 KiB, more than the shared-staging kernel gets
+    (48, 16256, 32, 4, "bf16"),
+    (33, 16288, 32, 8, "f16"),
+    (40, 27072, 64, 8, "bf16"),
+    (40, 27136, 64, 8, "f16"),
+    (17, 40576, 128, 8, "bf16"),
+    (5120, 17920, 32, 4, "bf16"),    # past it
+    (33, 81920, 64, 4, "bf16"),      # x past a workgroup's LDS
+    (20, 98304, 128, 8, "f16"),
+    (16, 80064, 64, 6, "bf16"),
+    (16, (1 << 21) + 64, 64, 4, "bf16"),
+])
+def test_one_long_row(device, oracle, n, k, gs, bits, dtype):
+    """Decode with K past what the layouts with x and constants in LDS take."""
+    _close(*_run(device, oracle, 1, n, k, gs, bits, dtype))
+
+
 @pytest.mark.parametrize("m", [1, 3])
 def test_decode_large_scales(device, oracle, m):
     """bf16 scales of 2^104 and above overflow the subnormal form."""
