@@ -108,8 +108,12 @@ hipError_t launch_qmm_tile_n(hipStream_t s, const TilePlan& p, void* scratch, co
 TilePlan qmm_tile_t_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
 hipError_t launch_qmm_tile_t(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,
                              void* y, int m, int n, int k);
-// transpose=false for what its tiles do not take: K = 0 (stores zeros), larger tables.
-hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
+// transpose=false for what its tiles do not take: K = 0 (stores zeros), longer K,
+// larger tables.  split > 1 splits K and needs qmm_n_scratch_bytes of fp32 partials.
+int qmm_n_split(int m, int n, int k, int cu_count);
+size_t qmm_n_scratch_bytes(int m, int n, int split);
+hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
+                        float* partial);
 // Decode (M = 1) transpose=false at 4/8 bits on the VALU: rows per thread
 // and step, K parts and the split-K scratch they need (arrival words at the
 // head, zero between launches, then fp32 sums); parts == 1 needs none.

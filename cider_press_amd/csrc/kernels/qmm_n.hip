@@ -11,7 +11,7 @@
 //
 // M > 1 (and M = 1 at the widths qvm does not take) runs on the tiles of
 // qmm_tile_n.hip; qmm_n_kernel keeps what those do not take: K = 0 (it stores
-// zeros) and tables past 31-bit byte offsets.
+// zeros), K past 2^21 and tables past 31-bit byte offsets.
 //
 // The MFMA operands want 8 consecutive k per lane, while a row of W is
 // contiguous along n.  Each K-step therefore dequantizes its 64 x 64 W tile
@@ -19,6 +19,10 @@
 // bit-exact chunk dequantizer) and writes it transposed into LDS ([n][k]);
 // the activation tile is staged as is ([m][k]).  Four waves then run
 // v_mfma_f32_16x16x32 on 32 x 32 quadrants of the 64 x 64 output tile.
+// Grids with few tiles split K over blockIdx.z: each part stores an fp32
+// partial tile, and a second kernel adds the parts in order (deterministic)
+// and rounds to T (one workgroup per tile walking 2^21 of K takes 42 ms, split
+// 0.7 ms: 4-bit, 8 x 512).
 #include <algorithm>
 
 #include "../cpq_internal.hpp"
@@ -37,7 +41,8 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
                                                     const uint16_t* __restrict__ scales,
                                                     const uint16_t* __restrict__ biases,
                                                     const uint16_t* __restrict__ x, uint16_t* __restrict__ y, int m,
-                                                    int n, int k, int gs_shift) {
+                                                    int n, int k, int gs_shift, int k_part,
+                                                    float* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) uint16_t xs[NT_M * NT_P];
   __shared__ __attribute__((aligned(16))) uint16_t wt[NT_N * NT_P];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -52,6 +57,7 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  const int k_lo = blockIdx.z * k_part, k_hi = min(k, k_lo + k_part);  // k_part % NT_K == 0
   // Raw inputs of one K-step, loaded a step ahead: two 8-k activation pieces
   // per thread, and for threads < 128 one 32-column weight chunk of one k row
   // with its (scale, bias).
@@ -66,11 +72,11 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
       const int i = tid + 256 * h;
       const int gm = m0 + (i >> 3), gk = k0 + 8 * (i & 7);
       xv[h] = u32x4{0u, 0u, 0u, 0u};
-      if (gm < m && gk < k) xv[h] = *reinterpret_cast<const u32x4*>(x + (size_t)gm * k + gk);
+      if (gm < m && gk < k_hi) xv[h] = *reinterpret_cast<const u32x4*>(x + (size_t)gm * k + gk);
     }
     if (tid < 2 * NT_K) {
       const int gk = k0 + kr;
-      if (gk < k && col < n) {
+      if (gk < k_hi && col < n) {
         load_chunk<BITS>(w + (size_t)gk * row_words, (size_t)(col >> 5), wv);
         const size_t gi = (size_t)gk * G + (size_t)(col >> gs_shift);
         sv = scales[gi];
@@ -82,8 +88,8 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
       }
     }
   };
-  if (k > 0) fetch(0);
-  for (int k0 = 0; k0 < k; k0 += NT_K) {
+  if (k_lo < k_hi) fetch(k_lo);
+  for (int k0 = k_lo; k0 < k_hi; k0 += NT_K) {
     // Stage the fetched step: activations as is, weights dequantized and
     // transposed into wt[n][k].
 #pragma unroll
@@ -101,7 +107,7 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
         dst[(2 * j + 1) * NT_P] = (uint16_t)(o[j] >> 16);
       }
     }
-    if (k0 + NT_K < k) fetch(k0 + NT_K);  // in flight during the MFMAs
+    if (k0 + NT_K < k_hi) fetch(k0 + NT_K);  // in flight during the MFMAs
     __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < NT_K; ks += 32) {
@@ -127,9 +133,26 @@ __global__ __launch_bounds__(256) void qmm_n_kernel(const uint32_t* __restrict__
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = m0 + wm + 16 * i + 4 * g + e;
-        if (row < m && col < n) y[(size_t)row * n + col] = TT::from_f32(acc[i][j][e]);
+        if (row < m && col < n) {
+          if (partial)
+            partial[((size_t)blockIdx.z * m + row) * n + col] = acc[i][j][e];
+          else
+            y[(size_t)row * n + col] = TT::from_f32(acc[i][j][e]);
+        }
       }
     }
+}
+
+// y = RNE_T(sum over parts p in order of partial[p]).
+template <typename TT>
+__global__ __launch_bounds__(256) void qmm_n_reduce_kernel(const float* __restrict__ partial, int parts, size_t mn,
+                                                           uint16_t* __restrict__ y) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mn; i += stride) {
+    float v = partial[i];
+    for (int p = 1; p < parts; ++p) v += partial[(size_t)p * mn + i];
+    y[i] = TT::from_f32(v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -330,30 +353,54 @@ hipError_t launch_qvm_rpt(hipStream_t s, const QvmPlan& p, void* scratch, const 
 }
 
 template <typename TT, int BITS>
-hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k) {
+hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
+                    float* partial) {
   int gs_shift = 0;
   while ((1 << gs_shift) < q.gs) ++gs_shift;
-  const dim3 grid((unsigned)((n + NT_N - 1) / NT_N), (unsigned)((m + NT_M - 1) / NT_M));
+  const int k_part = split > 1 ? (k / split + NT_K - 1) / NT_K * NT_K : (k + NT_K - 1) / NT_K * NT_K;
+  const int parts = split > 1 ? (k + k_part - 1) / k_part : 1;
+  const dim3 grid((unsigned)((n + NT_N - 1) / NT_N), (unsigned)((m + NT_M - 1) / NT_M), (unsigned)parts);
   hipLaunchKernelGGL((qmm_n_kernel<TT, BITS>), grid, dim3(256), 0, s, q.w, static_cast<const uint16_t*>(q.scales),
                      static_cast<const uint16_t*>(q.biases), static_cast<const uint16_t*>(x),
-                     static_cast<uint16_t*>(y), m, n, k, gs_shift);
+                     static_cast<uint16_t*>(y), m, n, k, gs_shift, k_part > 0 ? k_part : NT_K,
+                     parts > 1 ? partial : nullptr);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || parts <= 1) return e;
+  const size_t mn = (size_t)m * n;
+  size_t blocks = (mn + 255) / 256;
+  if (blocks > 256 * 16) blocks = 256 * 16;
+  hipLaunchKernelGGL((qmm_n_reduce_kernel<TT>), dim3((unsigned)blocks), dim3(256), 0, s, partial, parts, mn,
+                     static_cast<uint16_t*>(y));
   return hipGetLastError();
 }
 
 template <typename TT>
-hipError_t launch_bits(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k) {
+hipError_t launch_bits(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
+                       float* partial) {
   switch (q.bits) {
-    case 2: return launch_t<TT, 2>(s, q, x, y, m, n, k);
-    case 3: return launch_t<TT, 3>(s, q, x, y, m, n, k);
-    case 4: return launch_t<TT, 4>(s, q, x, y, m, n, k);
-    case 5: return launch_t<TT, 5>(s, q, x, y, m, n, k);
-    case 6: return launch_t<TT, 6>(s, q, x, y, m, n, k);
-    case 8: return launch_t<TT, 8>(s, q, x, y, m, n, k);
+    case 2: return launch_t<TT, 2>(s, q, x, y, m, n, k, split, partial);
+    case 3: return launch_t<TT, 3>(s, q, x, y, m, n, k, split, partial);
+    case 4: return launch_t<TT, 4>(s, q, x, y, m, n, k, split, partial);
+    case 5: return launch_t<TT, 5>(s, q, x, y, m, n, k, split, partial);
+    case 6: return launch_t<TT, 6>(s, q, x, y, m, n, k, split, partial);
+    case 8: return launch_t<TT, 8>(s, q, x, y, m, n, k, split, partial);
     default: return hipErrorInvalidValue;
   }
 }
 
 }  // namespace
+
+// Parts of K so that the grid has about two workgroups per CU, each part at
+// least two 64-deep K steps.
+int qmm_n_split(int m, int n, int k, int cu_count) {
+  const long tiles = (long)((n + NT_N - 1) / NT_N) * ((m + NT_M - 1) / NT_M);
+  const long want = 2L * (cu_count > 0 ? cu_count : 256);
+  int split = 1;
+  while (tiles * split * 2 <= want && k / (split * 2) >= 2 * NT_K) split *= 2;
+  return split;
+}
+
+size_t qmm_n_scratch_bytes(int m, int n, int split) { return split > 1 ? (size_t)split * m * n * 4 : 0; }
 
 // The decode kernel's plan: rows per thread and step (4; 2 when the
 // 4-row steps number more than four per CU, where shorter steps in a loop
@@ -410,10 +457,12 @@ hipError_t launch_qvm(hipStream_t s, const QvmPlan& p, void* scratch, const Quan
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k) {
+hipError_t launch_qmm_n(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k, int split,
+                        float* partial) {
   if (m == 0 || n == 0) return hipSuccess;  // K == 0 still runs: it stores zeros
-  if (q.dtype == CPQ_DTYPE_BF16) return launch_bits<BF16>(s, q, x, y, m, n, k);
-  if (q.dtype == CPQ_DTYPE_F16) return launch_bits<F16>(s, q, x, y, m, n, k);
+  if (split > 1 && !partial) return hipErrorInvalidValue;
+  if (q.dtype == CPQ_DTYPE_BF16) return launch_bits<BF16>(s, q, x, y, m, n, k, split, partial);
+  if (q.dtype == CPQ_DTYPE_F16) return launch_bits<F16>(s, q, x, y, m, n, k, split, partial);
   return hipErrorInvalidValue;
 }
 

@@ -800,7 +800,20 @@ cpq_status cpq_affine_qmm_n(cpq_commands* cmds, cpq_dtype dtype, const uint32_t*
   if (plan.cfg >= 0)
     return cpq::launched(cpq::launch_qmm_tile_n(cmds->stream, plan, cmds->scratch, q, x, y, (int)m, (int)n, (int)k),
                          "affine_qmm_n launch");
-  return cpq::launched(cpq::launch_qmm_n(cmds->stream, q, x, y, (int)m, (int)n, (int)k), "affine_qmm_n launch");
+  // What the tiles do not take: K split into fp32 partials in session scratch
+  // (past the arrival counters) when the session's scratch holds them, else no
+  // split (the choice depends on the shape and the session only).
+  int split = cpq::qmm_n_split((int)m, (int)n, (int)k, cmds->dev ? cmds->dev->cu_count : 0);
+  float* partial = nullptr;
+  if (split > 1) {
+    void* scratch = nullptr;
+    if (cpq::session_scratch(cmds, cpq::kWideCounterBytes + cpq::qmm_n_scratch_bytes((int)m, (int)n, split), &scratch))
+      partial = reinterpret_cast<float*>(static_cast<char*>(scratch) + cpq::kWideCounterBytes);
+    else
+      split = 1;
+  }
+  return cpq::launched(cpq::launch_qmm_n(cmds->stream, q, x, y, (int)m, (int)n, (int)k, split, partial),
+                       "affine_qmm_n launch");
 }
 
 cpq_status cpq_embed_tokens(cpq_commands* cmds, cpq_dtype dtype, const uint32_t* w_q, size_t w_q_len,

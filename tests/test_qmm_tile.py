@@ -2,6 +2,7 @@
 of tiles, K stages and groups, every width; scales too large for the
 subnormal form of the dequantization."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -57,6 +58,25 @@ def test_tile_n(device, library, oracle, monkeypatch, cfg, m, n, k, gs, bits, dt
     outs, ref = _run_n(device, library, oracle, m, n, k, gs, bits, dtype, calls=2)
     _close(outs[0], ref, dtype)
     assert np.array_equal(outs[0], outs[1])  # parts are added in k order whoever finishes last
+
+
+def test_long_k_n_is_split(device, library, oracle):
+    """K past the tiles' 31-bit ranges keeps its K split: a column tile
+    walking 2^21 of K unsplit take tens of milliseconds, split under one."""
+    m, n, k, gs, bits, dtype = 5, 32, (1 << 21) + 8, 32, 4, "bf16"
+    outs, ref = _run_n(device, library, oracle, m, n, k, gs, bits, dtype, calls=2)
+    _close(outs[0], ref, dtype)
+    assert np.array_equal(outs[0], outs[1])
+    W, S, B = (device.alloc_buffer(c, d) for c, d in ((k * n // 8, "u32"), (k * n // gs, dtype), (k * n // gs, dtype)))
+    X, Y, cmds = device.alloc_buffer(m * k, dtype), device.alloc_buffer(m * n, dtype), device.commands()
+    took = []
+    for _ in range(5):
+        cmds.commit_and_wait()
+        begin = time.perf_counter()
+        kqmm.affine_qmm_n(cmds, library, W, S, B, X, Y, m, n, k, gs, bits)
+        cmds.commit_and_wait()
+        took.append(time.perf_counter() - begin)
+    assert min(took) < 10e-3, took
 
 
 @pytest.mark.parametrize("split", [1, 2])
