@@ -7,7 +7,7 @@
 //
 // This kernel takes every shape and is the one for what the faster kernels
 // (qmm_dma.hip, qmm_tile_t.hip) leave: N not a multiple of 32 (one row only),
-// K past 2^21.
+// K past about 2^24.
 //
 // Tiling: a 256-thread workgroup owns a BM x BN output tile and walks K in
 // 32-element steps (one quantization chunk per W row, always inside one

@@ -52,9 +52,11 @@ struct Args {
 
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 
+constexpr uint64_t kRange = 0x7ffffff0ull;  // bytes addressed through one buffer at most
+
 __device__ __forceinline__ Rsrc rsrc(const void* p, uint64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0,
-                                           (int)(bytes > 0x7ffffff0ull ? 0x7ffffff0u : (uint32_t)bytes), 0x00020000);
+                                           (int)(bytes > kRange ? (uint32_t)kRange : (uint32_t)bytes), 0x00020000);
 }
 
 template <typename TT>
@@ -274,9 +276,12 @@ struct Shape {
 // The cheapest (tile, split) for m x n x k: rounds of workgroups, each its
 // stages plus about 4 us of launch, prologue and store; a split adds an
 // exchange of 1 us + 0.35 us per part + its parked bytes, written and read, at
-// about 4 TB/s.  cfg < 0 where nothing fits.  CPQ_TILE_CFG and CPQ_QMM_SPLIT
+// about 4 TB/s.  A tile's rows of X, and of W at w_bits per weight (0: addressed
+// some other way), lie within a buffer's 31-bit range.  cfg < 0 where nothing
+// fits.  CPQ_TILE_CFG and CPQ_QMM_SPLIT
 // force the tile and the split (test hooks, read per call).
-inline TilePlan plan_tiles(const Shape* shapes, int count, int m, int n, int k, int cu_count, size_t scratch_cap) {
+inline TilePlan plan_tiles(const Shape* shapes, int count, int m, int n, int k, int w_bits, int cu_count,
+                           size_t scratch_cap) {
   const long cus = cu_count > 0 ? cu_count : 256;
   const int S = (k + BK - 1) / BK;
   const int only = env_int("CPQ_TILE_CFG", -1), forced = env_int("CPQ_QMM_SPLIT", 0);
@@ -284,6 +289,7 @@ inline TilePlan plan_tiles(const Shape* shapes, int count, int m, int n, int k, 
   for (int c = 0; c < count; ++c) {
     if (only >= 0 && only < count && c != only) continue;
     const Shape& sh = shapes[c];
+    if ((uint64_t)std::max(16 * sh.bm, w_bits * sh.bn) * (uint64_t)k / 8 > kRange) continue;
     const long tiles = (long)((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn);
     int previous = 0;
     for (int want = 1; want <= 16; ++want) {

@@ -331,7 +331,7 @@ TilePlan qmm_tile_n_plan(const QuantArgs& q, int m, int n, int k, int cu_count, 
   if (m < 1 || k < 1 || k % 8 != 0 || n % 32 != 0 || k > (1 << 21) || n > (1 << 24) ||
       (uint64_t)k * (n / q.gs) * 2 >= 0x7ffffff0ull)
     return TilePlan{-1, 1, 0, 0.f};
-  return tile::plan_tiles(tile::kShapes, (int)(sizeof(tile::kShapes) / sizeof(tile::kShapes[0])), m, n, k, cu_count,
+  return tile::plan_tiles(tile::kShapes, (int)(sizeof(tile::kShapes) / sizeof(tile::kShapes[0])), m, n, k, 0, cu_count,
                           scratch_cap);
 }
 

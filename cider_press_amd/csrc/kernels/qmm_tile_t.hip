@@ -398,11 +398,11 @@ hipError_t launch_bits(int bits, int cfg, hipStream_t s, const Args& a) {
 }  // namespace tile
 
 TilePlan qmm_tile_t_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap) {
-  // 256 rows of X, of W and of the scale table within the 31-bit ranges of
-  // their buffers; 32 columns are stored together.
-  if (m < 1 || n < 32 || n % 32 != 0 || k < 32 || k > (1 << 21)) return TilePlan{-1, 1, 0, 0.f};
-  return tile::plan_tiles(tile::kShapes, (int)(sizeof(tile::kShapes) / sizeof(tile::kShapes[0])), m, n, k, cu_count,
-                          scratch_cap);
+  // 32 columns are stored together.  K past 2^21 leaves the smaller tiles, past
+  // about 2^24 none (4-bit 8 x 256, K = 2^21 + 1024: general kernel 58 ms, tiles 1.0).
+  if (m < 1 || n < 32 || n % 32 != 0 || k < 32) return TilePlan{-1, 1, 0, 0.f};
+  return tile::plan_tiles(tile::kShapes, (int)(sizeof(tile::kShapes) / sizeof(tile::kShapes[0])), m, n, k, q.bits,
+                          cu_count, scratch_cap);
 }
 
 hipError_t launch_qmm_tile_t(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,

@@ -149,6 +149,29 @@ def test_tile_t(device, library, oracle, tiles, cfg, m, n, k, gs, bits, dtype, s
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("m,n,k,gs,bits,dtype", [
+    (3, 32, (1 << 21) + 32, 32, 8, "bf16"),    # one past what 256 rows of X allow
+    (2, 32, (1 << 23) + 128, 128, 4, "f16"),   # the smallest tile only
+])
+def test_tile_t_long_k(device, library, oracle, m, n, k, gs, bits, dtype):
+    """K past 2^21 stays on the tiles (those whose rows fit 31-bit ranges), its
+    K split with it: the general kernel takes tens of milliseconds."""
+    outs, ref = _run_t(device, library, oracle, m, n, k, gs, bits, dtype, calls=2)
+    _close(outs[0], ref, dtype)
+    assert np.array_equal(outs[0], outs[1])
+    words, groups = k * n * bits // 32, k * n // gs
+    W, S, B = device.alloc_buffer(words, "u32"), device.alloc_buffer(groups, dtype), device.alloc_buffer(groups, dtype)
+    X, Y, cmds = device.alloc_buffer(m * k, dtype), device.alloc_buffer(m * n, dtype), device.commands()
+    took = []
+    for _ in range(5):
+        cmds.commit_and_wait()
+        begin = time.perf_counter()
+        kqmm.affine_qmm_t(cmds, library, W, S, B, X, Y, m, n, k, gs, bits)
+        cmds.commit_and_wait()
+        took.append(time.perf_counter() - begin)
+    assert min(took) < 20e-3, took
+
+
 def test_tile_t_skips_values_past_k(device, library, oracle, tiles):
     """The half stage past K holds the next row of X: an infinity there must
     not reach the row before it."""
