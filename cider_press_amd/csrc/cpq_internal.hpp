@@ -106,6 +106,7 @@ hipError_t launch_qmm_tile_n(hipStream_t s, const TilePlan& p, void* scratch, co
 // Y[M, N] = X[M, K] . dequant(W[N, K])^T on tiles, every width; N % 32 == 0,
 // K up to about 2^24 (a tile's rows within 31-bit ranges).
 TilePlan qmm_tile_t_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap);
+float qmm_tile_t_us(const QuantArgs& q, const TilePlan& p, int m, int n, int k, int cu_count);
 hipError_t launch_qmm_tile_t(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,
                              void* y, int m, int n, int k);
 // transpose=false for what its tiles do not take: K = 0 (stores zeros), longer K,

@@ -663,14 +663,17 @@ int qmm_dma_split(int m, int n, int k, int gs, int bits, int cu_count) {
   return best;
 }
 
-// Estimated time: the k-units of the split's makespan at 6.1 ns, and for a
-// split 2 us and its parked bytes (written and read, mostly through the L2 of
-// one XCD) at 16 TB/s.
+// Estimated time (us): rounds of one workgroup per CU, each 6 us and its k range
+// at 5.2 us per 1000, the chip's share of the stream at 2.2 us per 1000 and per
+// CU, and for a split 3 us and its parked bytes at 5 TB/s.  Against 639 measured
+// calls (33 .. 2100 rows, N 512 .. 40000, K 1024 .. 16384): 5th to 95th
+// percentile within 0.91 .. 1.08.
 float qmm_dma_us(int m, int n, int k, int split, int cu_count) {
   const long tiles = (long)((m + DBM - 1) / DBM) * ((n + DBN - 1) / DBN);
-  const long cus = cu_count > 0 ? cu_count : 256, rounds = (tiles * split + cus - 1) / cus;
-  const float us = 0.0061f * (float)(rounds * (k / split + 2000));
-  return split > 1 ? us + 2.f + 2.f * (float)(tiles * split * DPART * 4) / 16e6f : us;
+  const long cus = cu_count > 0 ? cu_count : 256, wgs = tiles * split, rounds = (wgs + cus - 1) / cus;
+  const float kk = (float)(k / split) * 1e-3f;
+  const float us = (float)rounds * (6.f + 5.2f * kk) + 2.2f * kk * (float)wgs / (float)cus;
+  return split > 1 ? us + 3.f + (float)wgs * (float)(DPART * 4) / 5e6f : us;
 }
 
 size_t qmm_dma_scratch_bytes(int m, int n, int split) {

@@ -9,6 +9,8 @@
 // traffic (2304 cycles per stage of a 256 x 256 tile against 2048 of MFMA)
 // bounded it.  Here a 256 x 256 tile moves 1280 cycles' worth, and the WM waves
 // of a column block repeat its dequantization: 4.5 VALU per MFMA.
+#include <algorithm>
+
 #include "qmm_tile.hpp"
 
 namespace cpq {
@@ -403,6 +405,25 @@ TilePlan qmm_tile_t_plan(const QuantArgs& q, int m, int n, int k, int cu_count, 
   if (m < 1 || n < 32 || n % 32 != 0 || k < 32) return TilePlan{-1, 1, 0, 0.f};
   return tile::plan_tiles(tile::kShapes, (int)(sizeof(tile::kShapes) / sizeof(tile::kShapes[0])), m, n, k, q.bits,
                           cu_count, scratch_cap);
+}
+
+// The plan's time as measured, to compare with other kernels' (the plan itself
+// only ranks tiles): a tile's calls take this share of their estimate, unsplit
+// and split (4-bit, 639 shapes: 5th to 95th percentile within 0.91 .. 1.14
+// after it), and where several workgroups share a CU the wider words cost more
+// per stage (5, 6 bits 1.5, 8 bits 1.45 times; 8-bit 3 x 20544 x 10336 79.8 us,
+// plan 47.8).
+float qmm_tile_t_us(const QuantArgs& q, const TilePlan& p, int m, int n, int k, int cu_count) {
+  static const float kMeasured[][2] = {{1.04f, 0.90f}, {0.90f, 0.83f}, {1.06f, 0.95f}, {0.97f, 0.87f}, {0.85f, 0.84f}};
+  const tile::Shape& sh = tile::kShapes[p.cfg];
+  const long cus = cu_count > 0 ? cu_count : 256;
+  const long tiles = (long)((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn);
+  const long load = (tiles * p.split + cus - 1) / cus, rounds = (load + sh.resident - 1) / sh.resident;
+  const int S = (k + tile::BK - 1) / tile::BK, per = (S + p.split - 1) / p.split;
+  const float wide = q.bits == 8 ? 1.45f : q.bits >= 5 ? 1.5f : 1.f;
+  const float alone = sh.alone * (float)rounds, each = sh.each * (float)load;
+  const float us = p.us + (float)per * (std::max(alone, each * wide) - std::max(alone, each));
+  return us * kMeasured[p.cfg][p.split > 1];
 }
 
 hipError_t launch_qmm_tile_t(hipStream_t s, const TilePlan& p, void* scratch, const QuantArgs& q, const void* x,

@@ -201,3 +201,45 @@ def test_tile_t_large_scales(device, library, oracle, tiles, split, value):
     outs, ref = _run_t(device, library, oracle, 70, 512, 256, 64, 4, "bf16", edit)
     _close(outs[0][:, [70]], ref[:, [70]], "bf16")
     _close(np.delete(outs[0], 70, axis=1), np.delete(ref, 70, axis=1), "bf16")
+
+
+def _graph_us(device, library, m, n, k, gs, bits, calls=20):
+    """us a call of affine_qmm_t: the best of a few replays of a graph of calls."""
+    words, groups = n * k * bits // 32, n * k // gs
+    W, S, B = (device.alloc_buffer(c, d) for c, d in ((words, "u32"), (groups, "bf16"), (groups, "bf16")))
+    X, Y, cmds = device.alloc_buffer(m * k, "bf16"), device.alloc_buffer(m * n, "bf16"), device.commands()
+
+    def encode():
+        for _ in range(calls):
+            kqmm.affine_qmm_t(cmds, library, W, S, B, X, Y, m, n, k, gs, bits)
+
+    encode()
+    cmds.commit_and_wait()
+    cmds.begin_capture()
+    encode()
+    graph = cmds.end_capture()
+    took = []
+    for _ in range(12):
+        begin = time.perf_counter()
+        graph.launch(cmds)
+        cmds.commit_and_wait()
+        took.append(time.perf_counter() - begin)
+    graph.close()
+    return min(took) / calls * 1e6
+
+
+@pytest.mark.parametrize("m,n,k,gs,bits,other", [
+    (607, 3456, 2048, 32, 4, {}),                             # two-wave kernel, tiles a quarter slower
+    (143, 11744, 2048, 32, 4, {}),
+])
+def test_tiles_only_where_they_are_faster(device, library, monkeypatch, m, n, k, gs, bits, other):
+    """The routed call takes no longer than the kernel the tiles compete with
+    (forced: the two-wave kernel by a split of one, the dense form by its
+    hook), with an allowance for timing that is half of what the tiles lose."""
+    routed = _graph_us(device, library, m, n, k, gs, bits)
+    for name, value in other.items():
+        monkeypatch.setenv(name, value)
+    if m > 64:
+        monkeypatch.setenv("CPQ_QMM_SPLIT", "1")  # a forced split the two-wave kernel takes
+    forced = _graph_us(device, library, m, n, k, gs, bits)
+    assert routed <= 1.12 * forced, (routed, forced)
