@@ -272,6 +272,7 @@ size_t gather_decode_lds(int rows_max, int k, int kw);
 // 4 waves or 1 (never 2), so that zero K-padding to the next multiple of 512
 // (zero weights, scales, biases and activations past the logical K) keeps
 // every wave's steps and leaves every output bit unchanged.
+float dense_small_us(const QuantArgs& q, int m, int n, int k, int cu_count);
 bool dense_small_supported(const QuantArgs& q, int m, int n, int k);
 hipError_t launch_dense_small(hipStream_t s, const QuantArgs& q, const void* x, void* y, int m, int n, int k,
                               bool pad_exact = false);

@@ -105,46 +105,45 @@ namespace cpq {
 namespace {
 
 // Estimated time (us) of the small-M kernel a shape would run on without the
-// tiles: the dense form (8-row passes; it slows down once the passes' weights
-// pass about 25M), the tiled small-M kernel (rounds of one workgroup per CU,
-// its K range; chunks of it restage activations), or the slab kernel (rounds of
-// 16-column slabs).  Fitted to calls of M = 2 .. 64 at (N, K) from 1152 to 12288;
-// within about 20 % where the choice is close.
+// tiles: the dense form (its own estimate), the tiled small-M kernel (all of K in
+// one workgroup up to 16 rows; past that rounds of one workgroup per CU, its K
+// range, chunks of it restaging activations), or the slab kernel (rounds of
+// 16-column slabs; 2 bits apart: half the time of the other widths).  Fitted to
+// calls of M = 2 .. 64, N 256 .. 26000, K 512 .. 26000.
 float small_m_us(const QuantArgs& q, const SmallPlan& sp, bool dense, int m, int n, int k, long cus) {
-  const float kf = (float)k / 1024.f;
-  if (dense) {
-    const float v = (float)((m + 7) / 8) * (float)n * (float)k * 1e-6f;
-    return 4.f + 0.13f * std::min(v, 25.f) + 0.33f * std::max(0.f, v - 25.f) + 0.92f * kf;
-  }
-  if (sp.split > 0 && sp.mb == 1) return 4.f + (q.bits == 8 ? 1.8f : 1.2f) * kf * std::max(1.f, (float)n / 4096.f);
+  const float kf = (float)k / 1024.f, wgs = (float)((n + 15) / 16), rounds = (float)(((n + 15) / 16 + cus - 1) / cus);
+  if (dense) return dense_small_us(q, m, n, k, (int)cus);
+  if (sp.split > 0 && sp.mb == 1)
+    return 3.3f + kf * rounds * ((q.bits == 8 ? 0.97f : 0.44f) + 0.027f * (float)m) +
+           0.18e-6f * (float)n * (float)k * (float)q.bits / 8.f;
   if (sp.split > 0) {
-    const long wgs = (long)((n + 16 * sp.mb - 1) / (16 * sp.mb)) * sp.split;
-    return 6.f + 1.1f * (float)sp.mb * kf / (float)sp.split * (float)((wgs + cus - 1) / cus) * (sp.nch > 1 ? 1.8f : 1.f) +
+    const long w = (long)((n + 16 * sp.mb - 1) / (16 * sp.mb)) * sp.split;
+    return 6.f + 1.1f * (float)sp.mb * kf / (float)sp.split * (float)((w + cus - 1) / cus) * (sp.nch > 1 ? 1.8f : 1.f) +
            (sp.split > 1 ? 3.f : 0.f);
   }
+  if (q.bits == 2 && m <= 16)
+    return 4.3f + kf * (0.3f + 0.5f * rounds + 0.6f * (float)m / 16.f * wgs / (float)cus) + 0.34f * rounds;
   const float passes = (float)((m + 15) / 16);
-  return (4.f + 1.9f * kf) * (float)(((n + 15) / 16 + cus - 1) / cus) * (1.f + 0.015f * (float)std::min(m, 16)) *
-         (1.f + 0.4f * (passes - 1.f));
+  return (4.f + 1.9f * kf) * rounds * (1.f + 0.015f * (float)std::min(m, 16)) * (1.f + 0.4f * (passes - 1.f));
 }
-
-}  // namespace
-
-namespace {
 
 // Up to 16 rows on the decode kernel for any K.  A workgroup holds its rows in
 // LDS: two per CU, or one where the grid is no larger than the chip.  Other
 // widths always, while staging M rows per 16 columns pays (6-bit M = 2 .. 16:
 // 3520 x 3520 9.6 .. 11.4 -> 5.8 .. 7.7 us, 1152 x 4352 13.5 .. 11.4 -> 5.6 ..
-// 7.8; 16 x 32000 x 1152 13.9 / 16.7).  4 bits: 2 x 3520 x 3520 6.8 -> 5.0, 8 x
+// 7.8; 16 x 32000 x 1152 13.9 / 16.7; 2 bits, whose slab kernel costs half: 11 x
+// 14752 x 3200 20.9 / 14.7).  4 bits: 2 x 3520 x 3520 6.8 -> 5.0, 8 x
 // 5120 x 2560 9.7 -> 6.9; short rows and, past 4 rows on few columns, K in
-// whole 256s stay (16 x 1152 x 4352 6.4 / 7.1).  8 bits: 2 x 2560 x 10048 14.5 ->
+// whole 256s stay (16 x 1152 x 4352 6.4 / 7.1), from 64 blocks on at any
+// rows while K gives a wave a part of its second batch (3 x 1184 x 8448 7.5 / 9.2).  8 bits: 2 x 2560 x 10048 14.5 ->
 // 11.7, 16 x 3520 x 3520 9.9 -> 7.6; many columns stay (32000 x 1152 12.4 / 13.4).
 bool decode_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
   if (!decode_fits(q, m, n, k, x)) return false;
   const long wgs = (n + 15) / 16;
   if ((size_t)m * (size_t)k * 2 > 72 * 1024 && wgs > 256) return false;
-  if (q.bits != 4 && q.bits != 8) return (long)m * wgs <= 16384;
+  if (q.bits != 4 && q.bits != 8) return (long)m * wgs <= (q.bits == 2 && k >= 2048 ? 8192 : 16384);
   if (q.bits == 8) return k >= 2048 && wgs <= 400;
+  if (k % 256 == 0 && k > 6144 && k <= 10240 && wgs >= 64 && wgs < 256) return false;
   return k > 1024 && wgs < 1024 && (m <= 4 || k % 256 != 0 || wgs >= 256) && (m <= 8 || k >= 2048 || wgs >= 256);
 }
 
@@ -219,7 +218,7 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
     const bool dense = dense_ok && small_wgs * 4 < cus;
     const float est = small_m_us(q, sp, dense, m, n, k, cus);
     TilePlan tp{-1, 1, 0, 0.f};
-    if (small_on && dense_env < 1 && est > 6.f) {  // no tile takes less
+    if (small_on && dense_env < 1 && est > 6.f) {  // a cheap way out: below it the tiles hardly win (one 64-deep stage takes 4.4)
       tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.plan_bytes);
       if (tp.scratch_bytes > ex.scratch_bytes) tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
     }
@@ -229,7 +228,7 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
     // kernel reads each activation slice from L2 per wave): 48 x 4096 x 11008
     // 102 -> 24 us, 60 x 9984 x 3520 91 -> 18, 24 x 3520 x 3520 14.8 -> 11.5,
     // 6-bit 16 x 2560 x 10048 29 -> 19; 32 x 4096 x 4096 stays (11.3 / 12.4).
-    if (tp.cfg >= 0 && tp.us < 0.92f * est)
+    if (tp.cfg >= 0 && qmm_tile_t_us(q, tp, m, n, k, (int)cus) < 0.92f * est)
       return launch_qmm_tile_t(ex.stream, tp, ex.scratch, q, x, y, m, n, k);
     if (dense) return launch_dense_small(ex.stream, q, x, y, m, n, k);
     if (sp.split > 0) return launch_qmm_small(ex.stream, sp, ex.scratch, q, x, y, m, n, k);

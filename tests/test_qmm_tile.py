@@ -231,6 +231,8 @@ def _graph_us(device, library, m, n, k, gs, bits, calls=20):
 @pytest.mark.parametrize("m,n,k,gs,bits,other", [
     (607, 3456, 2048, 32, 4, {}),                             # two-wave kernel, tiles a quarter slower
     (143, 11744, 2048, 32, 4, {}),
+    (3, 24064, 10592, 32, 4, {"CPQ_SMALL_DENSE": "1"}),       # the dense form, tiles half as slow again
+    (4, 22880, 4032, 64, 4, {"CPQ_SMALL_DENSE": "1"}),
 ])
 def test_tiles_only_where_they_are_faster(device, library, monkeypatch, m, n, k, gs, bits, other):
     """The routed call takes no longer than the kernel the tiles compete with
