@@ -951,14 +951,23 @@ hipError_t launch_t(hipStream_t s, const QuantArgs& q, const void* x, void* y, i
   // The decode kernel for any K takes every other width, and 4/8 bits where the
   // layouts above do not: 6-bit 2048 x 2048 5.9 -> 4.8 us, 2048 x 6144 15.8 ->
   // 7.5; 4-bit 3520 x 3520 5.7 -> 4.8, 9984 x 3520 11.2 -> 8.7; 8-bit 3520 x
-  // 3520 6.5 -> 5.5.  Past 48 steps of 128 (a second batch per wave) or 512
-  // column blocks the shared-staging kernel, where it fits, is as fast at 8 bits,
-  // and past 48 steps at 4-bit groups of 32 (2560 x 9984: 9.5 against 10.4).
+  // 3520 6.5 -> 5.5.  The shared-staging kernel, where it fits, keeps what it does
+  // better.  K in whole 256s, whose constants it loads in whole words, past 2304:
+  // the decode kernel has a few waves of one batch (2560: 5 of 12; 8-bit 507 x
+  // 3072 5.3 / 4.7), or two of which the second is mostly empty (4-bit 4672 x
+  // 7168 15.8 / 10.0, 5441 x 7680 15.7 / 10.2); one full batch a wave and few
+  // columns are the exception (512 x 5120 5.5 / 5.8), and at 4 bits long K on many
+  // columns (34585 x 14848 81 / 146).  At 8 bits and at 4-bit groups of 32 also
+  // everything past one batch a wave (2560 x 9984 9.5 / 10.4), at 8 bits 512 column
+  // blocks.
   // Where it does not fit, a prefill kernel on one row took 219 us against 29.5 at
   // 4-bit 5120 x 17920, groups of 32.
+  const long wgs = (n + 15) / 16;
   const bool one_batch = k <= 6144;
+  const bool whole = k % 256 == 0 && k > 2304 && !(k > 4096 && one_batch && wgs <= 256);
   if (decode_fits(q, 1, n, k, x) &&
-      (!shared || (BITS == 4 && (one_batch || q.gs > 32)) || (BITS == 8 && one_batch && (n + 15) / 16 < 512)))
+      (!shared || (BITS == 4 && (one_batch || q.gs > 32) && !(whole && (k <= 10240 || wgs < 512))) ||
+       (BITS == 8 && one_batch && wgs < 512 && !whole)))
     return launch_decode(s, q, x, y, 1, n, k);
   if (!shared) {
     // Rows past what either holds in LDS (K of about 75000): the decode kernel

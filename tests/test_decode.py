@@ -1,12 +1,14 @@
 """The decode kernel for any K (up to 16 rows, every width): edges of columns,
 128-k steps, groups and waves; scales too large for the subnormal form."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
 
 from cider_press_amd import _lib
 from cider_press_amd.kernels import _ptr
+from cider_press_amd.kernels import qmv as kqmv
 from cider_press_amd.synthetic import from_bits, make_weight, make_x, to_bits
 
 pytestmark = pytest.mark.gpu
@@ -92,6 +94,52 @@ def test_decode_large_scales(device, oracle, m):
     y, ref, dtype = _run(device, oracle, m, 64, 1280, 64, 6, "bf16", edit)
     for cols in ([5], [40], [c for c in range(64) if c not in (5, 40)]):
         _close(y[:, cols], ref[:, cols], dtype)
+
+
+@pytest.mark.parametrize("n,k,gs,bits,dtype", [
+    (200, 7168, 64, 4, "bf16"),      # waves with ranges of different lengths
+    (8200, 2816, 64, 4, "f16"),      # the same on 512 column blocks
+    (33, 20480, 128, 4, "bf16"),     # every wave whole batches
+    (40, 9984, 32, 4, "f16"),
+    (48, 9216, 64, 8, "bf16"),
+    (8200, 3520, 64, 8, "f16"),
+    (17, 20480, 128, 8, "bf16"),
+])
+def test_shared_staging(device, oracle, n, k, gs, bits, dtype):
+    """Decode shapes that stay on the shared-staging kernel."""
+    def edit(s, b):
+        s[::3, ::5] = 0  # zero scales: its exact form inside one workgroup
+
+    _close(*_run(device, oracle, 1, n, k, gs, bits, dtype, edit))
+
+
+def test_one_row_costs_as_its_neighbours(device, library):
+    """K = 7168 (7 x 1024) on a kernel of its own next to the lean layout's 8192:
+    a wave with a second, mostly empty batch made it take 1.8 times as long."""
+    def us(n, k, gs=64, calls=20):
+        W, S, B = (device.alloc_buffer(c, d) for c, d in ((n * k // 8, "u32"), (n * k // gs, "bf16"),
+                                                          (n * k // gs, "bf16")))
+        X, Y, cmds = device.alloc_buffer(k, "bf16"), device.alloc_buffer(n, "bf16"), device.commands()
+
+        def encode():
+            for _ in range(calls):
+                kqmv.affine_qmv(cmds, library, W, S, B, X, Y, k, gs, 4)
+
+        encode()
+        cmds.commit_and_wait()
+        cmds.begin_capture()
+        encode()
+        graph, took = cmds.end_capture(), []
+        for _ in range(12):
+            begin = time.perf_counter()
+            graph.launch(cmds)
+            cmds.commit_and_wait()
+            took.append(time.perf_counter() - begin)
+        graph.close()
+        return min(took) / calls * 1e6
+
+    odd, even = us(4672, 7168), us(4672, 8192)
+    assert odd <= 1.4 * even, (odd, even)
 
 
 def test_decode_skips_values_past_k(device, oracle):
