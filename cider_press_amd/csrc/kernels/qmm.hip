@@ -252,8 +252,8 @@ hipError_t zero_words(hipStream_t s, void* p, size_t n_words) {
 // for what neither takes.  Measured (4-bit gs64, two-wave kernel / best tile): M = 512, K =
 // 4096: N = 4096 28.9 / 31.6 us, N = 12288 67.5 / 62.8; M = 2048: N = 4096
 // 77.3 / 74.7, N = 12288 226 / 214, N = 4096 at K = 12288 (the two-wave kernel
-// then splits K in 4) 350 / 203.  CPQ_QMM_DMA=0 turns the two-wave kernel
-// off; CPQ_QMM_SPLIT forces the K split, on that kernel where it takes it
+// then splits K in 4) 350 / 203.  CPQ_QMM_DMA=0 turns the two-wave kernel off,
+// CPQ_QMM_TILES=0 the tiles; CPQ_QMM_SPLIT forces the K split, on that kernel where it takes it
 // (test hooks, read per call).
 QmmPlan qmm_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap) {
   const bool sb16 = ((reinterpret_cast<uintptr_t>(q.scales) | reinterpret_cast<uintptr_t>(q.biases)) & 15u) == 0;
@@ -268,7 +268,8 @@ QmmPlan qmm_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t s
   while (split > 1 && (!qmm_dma_fits(m, n, k, q.gs, q.bits, split) || qmm_dma_scratch_bytes(m, n, split) > scratch_cap))
     split /= 2;
   if (split == 1 && !qmm_dma_fits(m, n, k, q.gs, q.bits, 1)) split = 0;
-  const TilePlan tile = qmm_tile_t_plan(q, m, n, k, cu_count, scratch_cap);
+  const TilePlan tile = env_int("CPQ_QMM_TILES", 1) != 0 ? qmm_tile_t_plan(q, m, n, k, cu_count, scratch_cap)
+                                                       : TilePlan{-1, 1, 0, 0.f};
   if (split > 0 && (forced > 0 || tile.cfg < 0 ||
                     qmm_dma_us(m, n, k, split, cu_count) <= 1.03f * qmm_tile_t_us(q, tile, m, n, k, cu_count)))
     return QmmPlan{QmmKernel::Dma, split, qmm_dma_scratch_bytes(m, n, split), tile};

@@ -192,6 +192,8 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
   const bool rows_ok = rows_env != 0 && aligned16(x) && aligned16(q.w) && qmm_rows_supported(q, m, n, k);
   if (rows_ok && (rows_env == 1 || (m >= 2 && k <= 1024 && 2L * qmm_rows_workgroups(n) >= cus)))
     return launch_qmm_rows(ex.stream, q, x, y, m, n, k);
+  const int phased = env_int("CPQ_DECODE_PHASED", -1);  // 1 where it applies, 0 off (test hook)
+  if (phased == 1 && decode_phased_fits(q, m, n, k, x)) return launch_decode_phased(ex.stream, q, x, y, m, n, k);
   if (m <= skinny_max_m(q, n, k)) {
     const bool small_on = env_int("CPQ_SMALL_M", 1) != 0;
     const bool rows_on = env_int("CPQ_QMV_ROWS", 1) != 0;
@@ -202,8 +204,6 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
       if (sp.split > 0 && sp.scratch_bytes > ex.scratch_bytes)
         sp = qmm_small_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
     }
-    const int phased = env_int("CPQ_DECODE_PHASED", -1);  // 1 where it applies, 0 off (test hook)
-    if (phased == 1 && decode_phased_fits(q, m, n, k, x)) return launch_decode_phased(ex.stream, q, x, y, m, n, k);
     if (small_on && rows_on && qmv_rows_fits(q, m, n, k, x)) return launch_qmv_rows(ex.stream, q, x, y, m, n, k);
     if (small_on && dense_env < 1 && env_int("CPQ_TILE_CFG", -1) < 0 && decode_rows(q, m, n, k, x))
       return launch_decode(ex.stream, q, x, y, m, n, k);

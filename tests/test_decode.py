@@ -165,7 +165,7 @@ def test_decode_skips_values_past_k(device, oracle):
     (7, 64, 12288, 64, 8, "bf16", 0),     # two phases, whole
     (16, 96, 9632, 32, 5, "bf16", 1),     # 9 waves, a last phase of part of a batch, a last wave with fewer steps
     (12, 2080, 8064, 128, 8, "f16", 0),   # as the route takes it
-    (2, 32, 40960, 64, 4, "f16", 1),      # one row block, many batches a phase
+    (2, 32, 40960, 64, 4, "f16", 1),      # one row block, many batches a phase; more groups than the slab kernel holds
     (16, 32, 30720, 64, 2, "bf16", 0),    # many phases
 ])
 def test_decode_phased(device, oracle, monkeypatch, m, n, k, gs, bits, dtype, skew):

@@ -239,9 +239,9 @@ def test_qmv_capacity_rejected_before_launch(device, library):
     (33, 96, 256, 64, 2, "bf16"),
     (40, 64, 384, 32, 6, "bf16"),
     (2, 32, 128, 64, 4, "bf16"),
-    (96, 160, 4096, 32, 4, "f16"),         # staged kernel: 3-slot ring (128 groups), N and M tails
-    (136, 224, 2048, 64, 8, "f16"),        # staged kernel, 8-bit, f16
-    (256, 128, 12288, 128, 4, "bf16"),     # staged kernel, long K
+    (96, 160, 4096, 32, 4, "f16"),         # tiles: 128 groups a row, N and M tails
+    (136, 224, 2048, 64, 8, "f16"),        # tiles, 8-bit, f16
+    (256, 128, 12288, 128, 4, "bf16"),     # tiles, long K
 ])
 def test_qmm_t_parity(device, library, oracle, m, n, k, gs, bits, dtype):
     rng = np.random.default_rng(m * 7 + n + bits)
@@ -264,9 +264,15 @@ def test_quantized_matmul_routes_all_m(device, library, oracle, m, bits, gs):
     assert_tol(oracle, y, ref, x, k, "bf16", f"routed m={m}")
 
 
-# Routed small-M shapes (up to 64 rows while N <= 8192) across the three
-# small-M kernels: the decode layout with M rows, the tiled small-M kernel and
-# the slab kernel.
+def _slab_only(monkeypatch):
+    """Up to 64 rows on the slab kernel, whatever the route would choose."""
+    for name in ("CPQ_SMALL_M", "CPQ_SMALL_DENSE", "CPQ_SMALL_ROWS"):
+        monkeypatch.setenv(name, "0")
+
+
+# Small-M shapes (up to 64 rows while N <= 8192) as routed and on the slab
+# kernel, whose wave counts and slabs per workgroup they cover.
+@pytest.mark.parametrize("slab", [False, True])
 @pytest.mark.parametrize("m,n,k,bits,gs", [
     (5, 8192, 1024, 4, 64),     # 1 row block, 4 waves (512 slabs)
     (20, 8192, 1024, 8, 64),    # 2 row blocks, 4 waves
@@ -276,7 +282,9 @@ def test_quantized_matmul_routes_all_m(device, library, oracle, m, bits, gs):
     (48, 8192, 256, 4, 64),     # two slabs, three row blocks
     (36, 8192, 512, 8, 32),     # two slabs, 8-bit, a ragged row block
 ])
-def test_small_m_wave_counts(device, library, oracle, m, n, k, bits, gs):
+def test_small_m_wave_counts(device, library, oracle, monkeypatch, m, n, k, bits, gs, slab):
+    if slab:
+        _slab_only(monkeypatch)
     rng = np.random.default_rng(m + n + k)
     w_q, s, b = make_weight(rng, n, k, gs, bits, "bf16")
     x = make_x(rng, m, k, "bf16")
@@ -290,7 +298,8 @@ def test_small_m_wave_counts(device, library, oracle, m, n, k, bits, gs):
     (40, 128, 12288, 32),   # 64-row blocks at the same size
     (3, 64, 40960, 32),     # constants would not fit in LDS: the prefill path takes it
 ])
-def test_small_m_long_k(device, library, oracle, m, n, k, gs):
+def test_small_m_long_k(device, library, oracle, monkeypatch, m, n, k, gs):
+    _slab_only(monkeypatch)
     rng = np.random.default_rng(m + k)
     w_q, s, b = make_weight(rng, n, k, gs, 4, "bf16")
     x = make_x(rng, m, k, "bf16")
@@ -314,22 +323,25 @@ def test_gather_per_slab_long_k(device, library, oracle):
 
 # The 4-bit prefill path runs the two-waves-per-SIMD kernel ("dma": 128 x 128
 # tiles, both operands streamed into LDS, K split over 1, 2 or 4 workgroups,
-# partial tiles summed by the last to finish), else the one-wave wide-tile
-# kernel ("wide"), else the staged kernel.  CPQ_QMM_SPLIT forces the split,
-# CPQ_QMM_DMA=0 / CPQ_QMM_WIDE=0 turn the first two off.
-_KERNEL_ENV = {"dma": ("1", "1"), "wide": ("0", "1"), "staged": ("0", "0")}
+# partial tiles summed by the last to finish) or the tiles of every width
+# ("tiles"), and what neither takes the general kernel ("general").
+# CPQ_QMM_SPLIT forces the split, CPQ_QMM_DMA=0 / CPQ_QMM_TILES=0 turn the first
+# two off.
+_KERNEL_ENV = {"dma": ("1", "1"), "tiles": ("0", "1"), "general": ("0", "0")}
 
 
 def _use_kernel(monkeypatch, kern):
-    dma, wide = _KERNEL_ENV[kern]
+    dma, tiles = _KERNEL_ENV[kern]
     monkeypatch.setenv("CPQ_QMM_DMA", dma)
-    monkeypatch.setenv("CPQ_QMM_WIDE", wide)
+    monkeypatch.setenv("CPQ_QMM_TILES", tiles)
+    for name in ("CPQ_SMALL_ROWS", "CPQ_SMALL_DENSE"):
+        monkeypatch.setenv(name, "0")
     # affine_qmm_t sends small M to the small-M kernels; these tests force
     # the prefill kernels at every M.
     monkeypatch.setenv("CPQ_SKINNY_MAX_M", "1")
 
 
-@pytest.mark.parametrize("kern", ["dma", "wide"])
+@pytest.mark.parametrize("kern", ["dma", "tiles"])
 @pytest.mark.parametrize("m,n,k,gs,dtype,split", [
     (256, 512, 2048, 64, "bf16", 1),
     (256, 512, 2048, 64, "bf16", 2),
@@ -341,7 +353,7 @@ def _use_kernel(monkeypatch, kern):
     (129, 256, 2048, 128, "bf16", 2),
     (64, 4096, 4096, 64, "bf16", 4),       # config 4 at M = 64
 ])
-def test_qmm_wide_parity(device, library, oracle, monkeypatch, m, n, k, gs, dtype, split, kern):
+def test_qmm_split_parity(device, library, oracle, monkeypatch, m, n, k, gs, dtype, split, kern):
     _use_kernel(monkeypatch, kern)
     monkeypatch.setenv("CPQ_QMM_SPLIT", str(split))
     rng = np.random.default_rng(m + n + split)
@@ -359,7 +371,7 @@ def test_qmm_wide_parity(device, library, oracle, monkeypatch, m, n, k, gs, dtyp
 _SLOW_SB = {"bf16": (0x3000, 0x3C23), "f16": (0x0001, 0x211F)}
 
 
-_KERNEL_SPLITS = [("dma", 2), ("dma", 1), ("wide", 2), ("wide", 1), ("staged", 1)]
+_KERNEL_SPLITS = [("dma", 2), ("dma", 1), ("tiles", 2), ("tiles", 1), ("general", 1)]
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
@@ -376,6 +388,25 @@ def test_qmm_mixed_fast_and_slow_tiles(device, library, oracle, monkeypatch, dty
     y = run_qmm(device, library, w_q, s, b, x, m, n, k, gs, 4, dtype)
     ref = oracle.qmm_ref(x, w_q, s, b, m, n, k, gs, 4, dtype)
     assert_tol(oracle, y, ref, x, k, dtype, f"mixed {kern} split={split}")
+
+
+@pytest.mark.parametrize("m,n,k,gs,bits,dtype", [
+    (3, 64, 96, 32, 4, "bf16"),       # three 32-k steps, one row tile
+    (129, 160, 1024, 64, 8, "f16"),   # one past a tile of rows, a partial tile of columns
+    (200, 288, 352, 32, 6, "bf16"),
+    (70, 96, 640, 128, 3, "f16"),
+    (65, 128, 704, 64, 2, "bf16"),
+    (64, 32, 416, 32, 5, "bf16"),
+    (2048, 4128, 64, 32, 4, "bf16"),  # enough tiles for 128 rows a workgroup
+])
+def test_qmm_general_parity(device, library, oracle, monkeypatch, m, n, k, gs, bits, dtype):
+    _use_kernel(monkeypatch, "general")
+    rng = np.random.default_rng(m + n + k)
+    w_q, s, b = make_weight(rng, n, k, gs, bits, dtype)
+    x = make_x(rng, m, k, dtype)
+    y = run_qmm(device, library, w_q, s, b, x, m, n, k, gs, bits, dtype)
+    ref = oracle.qmm_ref(x, w_q, s, b, m, n, k, gs, bits, dtype, threads=8)
+    assert_tol(oracle, y, ref, x, k, dtype, f"general {m}x{n}x{k}")
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
@@ -400,8 +431,8 @@ def test_qmm_zero_scales_and_biases(device, library, oracle, monkeypatch, dtype,
     assert_tol(oracle, y, ref, x, k, dtype, f"zeros {kern} split={split}")
 
 
-@pytest.mark.parametrize("kern", ["dma", "wide"])
-def test_qmm_wide_split_is_deterministic(device, library, oracle, monkeypatch, kern):
+@pytest.mark.parametrize("kern", ["dma", "tiles"])
+def test_qmm_split_is_deterministic(device, library, oracle, monkeypatch, kern):
     """The split-K sum adds the parts in k order whatever order the
     workgroups finish in: repeated calls give identical bits."""
     _use_kernel(monkeypatch, kern)
@@ -421,7 +452,7 @@ def test_qmm_wide_split_is_deterministic(device, library, oracle, monkeypatch, k
         outs.append(Y.to_numpy())
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
     ref = oracle.qmm_ref(x, w_q, s, b, m, n, k, gs, 4, "bf16")
-    assert_tol(oracle, outs[0].reshape(m, n), ref, x, k, "bf16", "wide split=4")
+    assert_tol(oracle, outs[0].reshape(m, n), ref, x, k, "bf16", f"{kern} split=4")
 
 
 def test_qmm_rejects_unaligned_n(device, library):

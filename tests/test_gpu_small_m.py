@@ -145,9 +145,12 @@ def test_decode_layout_rows_parity(device, oracle, m, n, k, bits, gs, dtype):
     (33, 2048, 1152, 8, 128),
     (64, 8192, 512, 2, 32),
 ])
-def test_slab_kernel_parity(device, oracle, m, n, k, bits, gs):
-    """Shapes the tiled small-M kernels do not take run the slab kernel (one
-    16-column slab of W per workgroup, up to 64 rows per pass)."""
+def test_slab_kernel_parity(device, oracle, monkeypatch, m, n, k, bits, gs):
+    """The slab kernel (one 16-column slab of W per workgroup, up to 64 rows
+    per pass) at shapes the tiled small-M kernels do not take; the other
+    kernels that may be chosen for them are off."""
+    for name in ("CPQ_SMALL_M", "CPQ_SMALL_DENSE", "CPQ_SMALL_ROWS"):
+        monkeypatch.setenv(name, "0")
     rng = np.random.default_rng(m * 5 + n + k + bits)
     w_q, s, b = make_weight(rng, n, k, gs, bits, "bf16")
     x = make_x(rng, m, k, "bf16")
