@@ -304,10 +304,12 @@ __global__ __launch_bounds__(64 * MAXW) void decode_kernel(const uint32_t* __res
 // a wave's loads in flight at once), up to 12 waves, up to 8 where the grid
 // fills the chip twice (6-bit, us at 4 / 8 / 12 waves: 2048 x 2048 4.8 / 5.6 /
 // 5.6, 2048 x 6144 9.8 / 9.9 / 7.5, 9984 x 3520 4-bit 9.5 / 8.7 / 11.2).
+// CPQ_DECODE_WAVES sets their limit, 1 .. 12 (test hook).
 void decode_split(int n, int k, int* waves, int* steps) {
   const int S = (k + STEP - 1) / STEP;
   const int most = (n + 15) / 16 >= 512 ? 8 : MAXW;
-  const int w = std::min(env_int("CPQ_DECODE_WAVES", most), (S + BATCH - 1) / BATCH);
+  const int limit = std::max(1, std::min(MAXW, env_int("CPQ_DECODE_WAVES", most)));
+  const int w = std::min(limit, (S + BATCH - 1) / BATCH);
   *steps = (S + w - 1) / w;
   *waves = (S + *steps - 1) / *steps;
 }

@@ -47,7 +47,7 @@ def _close(y, ref, dtype):
     assert np.linalg.norm(y - ref) <= bound * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("waves", [1, 3, 12])
+@pytest.mark.parametrize("waves", [0, 1, 3, 12, 40])  # out of range: the nearest
 @pytest.mark.parametrize("m,n,k,gs,bits,dtype,skew", [
     (1, 1, 32, 32, 6, "bf16", 0),        # one column, a quarter step
     (1, 17, 96, 32, 3, "f16", 1),        # one column past a block, tables on an odd element
