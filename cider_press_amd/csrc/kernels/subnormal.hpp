@@ -7,9 +7,10 @@
 // with one rounding.  s * 2^(24 - p) is exact in fp32 for every f16 scale and
 // for every bf16 scale with a biased exponent below 231 (|s| < 2^104); larger
 // ones (and Inf, NaN) overflow, so callers compare the scales they meet with
-// kSubScaleLimit and use BigCst for them.  Compared on an MI355X with fmaf(s, q, b) over all
-// 65536 scale patterns of either type x 64 biases x q = 0..255: no
-// difference outside that range.  Against the 1024 + q form of
+// kSubScaleLimit and use BigCst for them.  Checked on the host for every scale
+// pattern, value and place (tests/test_subnormal.py); the fields' extraction on
+// the GPU against the oracle's weights, bit for bit, for every width
+// (tests/test_exact_weights.py).  Against the 1024 + q form of
 // dequant_slice_nat this needs no group check up front and no b - 1024 s.
 #pragma once
 

@@ -39,11 +39,14 @@ def _run(device, oracle, m, n, k, gs, bits, dtype, edit=None, skew=0):
 
 
 def _close(y, ref, dtype):
-    """Rounding the output to T moves each value by at most T's unit roundoff
-    (2^-8 with bf16's 8 significant bits, 2^-11 with f16's 11); fp32 sums of K
-    terms add a few 2^-24 of the terms' magnitude, here under 1e-5 of the norm."""
+    """Rounding to T errs by at most u of a value (2^-8 with bf16's 8 significant
+    bits, 2^-11 with f16's 11), and evenly up to there over many values: their
+    root mean square is at most u / sqrt(3).  fp32 sums of K terms add
+    2^-24 of partial sums as large as the result at random: under 1e-4 for the
+    bf16 cases' K (up to 2^21), 1e-5 for the f16 ones'."""
     assert np.isfinite(y).all()
-    bound = (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) + 1e-5
+    u = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -11
+    bound = u / (np.sqrt(3.0) if ref.size >= 256 else 1.0) + (1e-5 if dtype == "f16" else 1e-4)
     assert np.linalg.norm(y - ref) <= bound * np.linalg.norm(ref)
 
 
