@@ -282,31 +282,40 @@ struct Shape {
 // force the tile and the split (test hooks, read per call).
 inline TilePlan plan_tiles(const Shape* shapes, int count, int m, int n, int k, int w_bits, int cu_count,
                            size_t scratch_cap) {
-  const long cus = cu_count > 0 ? cu_count : 256;
-  const int S = (k + BK - 1) / BK;
+  const int cus = cu_count > 0 ? cu_count : 256, S = (int)(((unsigned)k + BK - 1) / BK);
   const int only = env_int("CPQ_TILE_CFG", -1), forced = env_int("CPQ_QMM_SPLIT", 0);
+  // The splits worth a look (no empty part, two stages at least) and their stages.
+  // Every op that may take a tile comes here: 32-bit divisions, and few.
+  int splits[16], pers[16], ways = 0;
+  for (int want = 1; want <= 16; ++want) {
+    if (forced > 0 && want != std::min(forced, 16)) continue;
+    const int per = (S + want - 1) / want, split = (S + per - 1) / per;
+    if (split > 1 && per < 2 && forced <= 0) break;
+    if (ways && split == splits[ways - 1]) continue;
+    splits[ways] = split;
+    pers[ways++] = per;
+  }
   TilePlan best{-1, 1, 0, 0.f};
   for (int c = 0; c < count; ++c) {
     if (only >= 0 && only < count && c != only) continue;
     const Shape& sh = shapes[c];
     if ((uint64_t)std::max(16 * sh.bm, w_bits * sh.bn) * (uint64_t)k / 8 > kRange) continue;
-    const long tiles = (long)((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn);
-    int previous = 0;
-    for (int want = 1; want <= 16; ++want) {
-      if (forced > 0 && want != std::min(forced, 16)) continue;
-      const int per = (S + want - 1) / want, split = (S + per - 1) / per;  // no empty part
-      if (split == previous || (split > 1 && per < 2 && forced <= 0)) continue;
-      previous = split;
-      if (tiles * split > (1L << 30)) continue;
+    const long all = (long)(((unsigned)m + sh.bm - 1) / (unsigned)sh.bm) * (long)(((unsigned)n + sh.bn - 1) / (unsigned)sh.bn);
+    if (all > (1L << 30)) continue;
+    const unsigned tiles = (unsigned)all;
+    for (int i = 0; i < ways; ++i) {
+      const int split = splits[i], per = pers[i];
       size_t bytes = 0;
       float us = 0.f;
       if (split > 1) {
+        if (tiles > (unsigned)kMaxTiles) break;
         const size_t parts = (size_t)tiles * split * sh.bm * sh.bn * sizeof(float);
         bytes = kWideCounterBytes + parts;
-        if (tiles > kMaxTiles || bytes > scratch_cap) continue;
+        if (bytes > scratch_cap) break;
         us = 1.f + 0.35f * (float)split + 2.f * (float)parts / 4e6f;
       }
-      const long load = (tiles * split + cus - 1) / cus, rounds = (load + sh.resident - 1) / sh.resident;
+      const unsigned load = (tiles * (unsigned)split + (unsigned)cus - 1) / (unsigned)cus;
+      const unsigned rounds = (load + (unsigned)sh.resident - 1) / (unsigned)sh.resident;
       us += (float)per * std::max(sh.alone * (float)rounds, sh.each * (float)load) + 3.f + (float)rounds;
       if (best.cfg < 0 || us < best.us) best = TilePlan{c, split, bytes, us};
     }
