@@ -207,9 +207,6 @@ QmmPlan qmm_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t s
 hipError_t launch_qmm(hipStream_t s, const QmmPlan& plan, void* scratch, const QuantArgs& q, const void* x,
                       void* y, int m, int n, int k);
 
-// qmm_plan + launch_qmm on a session (its stream, CU count and scratch).
-hipError_t launch_session_qmm(cpq_commands* cmds, const QuantArgs& q, const void* x, void* y, int m, int n, int k);
-
 // Where a matmul runs: stream, CU count, the split-K scratch at hand and the
 // capacity plans are made for (plans needing more than scratch_bytes are
 // remade for scratch_bytes).

@@ -5,8 +5,9 @@
 // kernels/quantized.h:749-975).  Each weight is dequantized to T (RNE of
 // fmaf(s, q, b)), products accumulate in fp32, one rounding to T.
 //
-// The lean layout of qmv.hip takes 4/8 bits at K in whole 512s; this kernel
-// takes the rest.  What it avoids is a chain of dependent waits: the
+// One row at 4/8 bits shares this with qmv.hip (its lean layout, K in whole
+// 512s, and its shared staging, some K in whole 256s); every other width is its
+// own.  What it avoids is a chain of dependent waits: the
 // dequantization through f16 subnormals needs no look at the constants before
 // the stream starts, so a wave issues its activations, constants and first
 // weights together, and waits for the rest of the workgroup only to add the
@@ -17,8 +18,9 @@
 // 4 step + g of its column (BITS words) and feeds it as four MFMA 16x16x32
 // operands (W's k order is permuted inside the step; the activations follow):
 //   x: the wave's range of each row in LDS (in phases where the workgroup's
-//      rows exceed it: a wave refills its own part, no barrier), a step's 16-byte pieces of row r at
-//      p ^ swz_key(r) (conflict-free for ds_read_b128's lane groups);
+//      rows exceed it: a wave refills its own part, no barrier), a step's
+//      16-byte pieces of row r at p ^ swz_key(r) (conflict-free for
+//      ds_read_b128's lane groups);
 //   scales, biases: the 4 steps' groups of a column read as aligned words
 //      around them and shifted (rows of group counts start on any 2 bytes);
 //   4 steps in flight, the next 4 requested before they are used.
@@ -34,33 +36,9 @@ namespace {
 using namespace dev;
 
 constexpr int STEP = 128, BATCH = 4, MAXW = 12;
-typedef __amdgpu_buffer_rsrc_t Rsrc;
 
 __device__ __forceinline__ Rsrc range(const void* p, uint64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
-}
-
-template <int BITS>
-__device__ __forceinline__ void load_chunk_words(Rsrc r, uint32_t off, uint32_t* w) {
-  if constexpr (BITS == 2) {
-    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-    w[0] = v.x; w[1] = v.y;
-  } else if constexpr (BITS == 3) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-    w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
-  } else {
-    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-    if constexpr (BITS == 5) w[4] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
-    if constexpr (BITS == 6) {
-      const u32x2 u = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off + 16, 0, 0));
-      w[4] = u.x; w[5] = u.y;
-    }
-    if constexpr (BITS == 8) {
-      const u32x4 u = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
-      w[4] = u.x; w[5] = u.y; w[6] = u.z; w[7] = u.w;
-    }
-  }
 }
 
 // The words holding a table's groups of BATCH steps, one more for the skew.
@@ -125,7 +103,7 @@ __device__ __forceinline__ void load_batch(const Geom& q, int t0, Batch<BITS, GS
   load_cst<GS_SHIFT>(q.br, q.boff + t0 * GB, p.b);
 #pragma unroll
   for (int j = 0; j < BATCH; ++j)
-    load_chunk_words<BITS>(q.wr, q.woff + (uint32_t)(t0 + j) * (4 * 4 * BITS), p.w[j]);
+    load_words<BITS>(q.wr, q.woff + (uint32_t)(t0 + j) * (4 * 4 * BITS), p.w[j]);
 }
 
 // One step.  A chunk past the row's end gets zero constants: zero weights (its

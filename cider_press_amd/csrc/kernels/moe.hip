@@ -156,7 +156,7 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const void* __restrict
   __shared__ uint32_t pick_of[ROWS];
   __shared__ uint32_t start[kMaxExperts];
   __shared__ uint32_t wave_total[16];
-  __shared__ uint8_t cnt[RW][kMaxExperts];
+  __shared__ __attribute__((aligned(4))) uint8_t cnt[RW][kMaxExperts];  // cleared by words
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rows = tokens * top_k;
   for (int i = tid; i < RW * kMaxExperts / 4; i += 1024) reinterpret_cast<uint32_t*>(&cnt[0][0])[i] = 0u;
@@ -254,9 +254,10 @@ __global__ __launch_bounds__(1024) void sort_scan_kernel(uint32_t* __restrict__ 
 }
 
 // Four waves per block of kSortRows rows, wave w on rows 64w .. 64w+63 of
-// the block; the last lane of each (wave, expert) run publishes the run's length, and a lane's sorted position
-// is its block's start for the expert, plus the counts of the earlier waves,
-// plus its rank -- so equal experts keep row order.
+// the block; the last lane of each (wave, expert) run publishes the run's
+// length, and a lane's sorted position is its block's start for the expert, plus
+// the counts of the earlier waves, plus its rank -- so equal experts keep row
+// order.
 __global__ __launch_bounds__(256) void sort_scatter_kernel(const uint32_t* __restrict__ experts, int rows, int top_k,
                                                            int n_experts, const uint32_t* __restrict__ starts,
                                                            uint32_t* __restrict__ lhs, uint32_t* __restrict__ rhs,

@@ -50,8 +50,6 @@ struct Args {
   unsigned int* counters;
 };
 
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-
 constexpr uint64_t kRange = 0x7ffffff0ull;  // bytes addressed through one buffer at most
 
 __device__ __forceinline__ Rsrc rsrc(const void* p, uint64_t bytes) {
@@ -96,29 +94,6 @@ __device__ __forceinline__ int row_key(int r) { return (r >> 1) & 7; }
 // Vector-memory instructions that load a chunk's words.
 template <int BITS>
 constexpr int kWordLoads = BITS >= 5 ? 2 : 1;
-
-template <int BITS>
-__device__ __forceinline__ void load_words(Rsrc r, uint32_t off, uint32_t* w) {
-  if constexpr (BITS == 2) {
-    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-    w[0] = v.x; w[1] = v.y;
-  } else if constexpr (BITS == 3) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-    w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
-  } else {
-    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-    if constexpr (BITS == 5) w[4] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
-    if constexpr (BITS == 6) {
-      const u32x2 u = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off + 16, 0, 0));
-      w[4] = u.x; w[5] = u.y;
-    }
-    if constexpr (BITS == 8) {
-      const u32x4 u = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
-      w[4] = u.x; w[5] = u.y; w[6] = u.z; w[7] = u.w;
-    }
-  }
-}
 
 // Keeps the operand reads ahead of the MFMAs they are to hide behind (left
 // alone, the compiler sinks them next to their uses).

@@ -289,9 +289,9 @@ hipError_t launch_n(hipStream_t st, const Args& a) {
 }
 
 
-// Stage times at 4-bit, group size 64.  With X in 32-bit LDS rows and W
-// dequantized by the workgroup, the widest tile costs least per multiply and
-// the narrowest starts most workgroups.
+// Stage times at 4-bit, group size 64.  A workgroup dequantizes each weight once
+// and stages both operands: the widest tile costs least per multiply, the
+// narrowest starts most workgroups.
 const Shape kShapes[] = {
     {256, 256, 1, 1.48f, 1.75f}, {128, 256, 1, 0.98f, 1.20f}, {128, 128, 2, 0.78f, 0.58f},
     {64, 128, 3, 0.68f, 0.42f},  {32, 128, 4, 0.55f, 0.38f},

@@ -19,6 +19,32 @@
 namespace cpq {
 namespace dev {
 
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+
+// The words of the chunk at byte `off` (4-byte aligned).
+template <int BITS>
+__device__ __forceinline__ void load_words(Rsrc r, uint32_t off, uint32_t* w) {
+  if constexpr (BITS == 2) {
+    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    w[0] = v.x; w[1] = v.y;
+  } else if constexpr (BITS == 3) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+    w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
+  } else {
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    if constexpr (BITS == 5) w[4] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
+    if constexpr (BITS == 6) {
+      const u32x2 u = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off + 16, 0, 0));
+      w[4] = u.x; w[5] = u.y;
+    }
+    if constexpr (BITS == 8) {
+      const u32x4 u = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
+      w[4] = u.x; w[5] = u.y; w[6] = u.z; w[7] = u.w;
+    }
+  }
+}
+
 // Largest scale pattern (sign cleared) that SubCst takes, plus one.
 template <typename TT>
 constexpr uint32_t kSubScaleLimit = Sig16<TT>::bf16 ? 231u << 7 : 0x10000u;

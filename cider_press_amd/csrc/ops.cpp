@@ -24,17 +24,15 @@ bool kernel_available(cpq_dtype dtype, uint32_t group_size, uint32_t bits) {
   return t_ok && gs_ok && b_ok;
 }
 
-// Largest M the routed op sends to the small-M kernels (the decode layout for
-// up to 16 rows, the tiled small-M kernel, or the slab kernel; see
-// cpq_quantized_matmul).  Up to 32 rows they always win; at 33..64 rows they
-// win while the prefill kernel's 128-wide tiles leave most CUs idle (N <=
-// 8192) and lose once N fills the chip (slab kernel 58 vs 31 us at N =
-// 12288).  CPQ_SKINNY_MAX_M overrides it, read once per process.  Shapes
-// whose slab constants do not fit in LDS (K / gs beyond about 500 groups per
-// row) never take them.
+// Largest M that may run on the small-M kernels (launch_matmul chooses among
+// them and the prefill tiles): 32, and 64 while N <= 8192, where the prefill
+// kernels' wide tiles leave most CUs idle (slab kernel 58 vs 31 us at N =
+// 12288).  CPQ_SKINNY_MAX_M overrides it (test hook).  Shapes whose slab
+// constants do not fit in LDS (K / gs beyond about 500 groups per row) never
+// take them.
 int skinny_max_m(const QuantArgs& q, int n, int k) {
   if (!skinny_fits(k, (int)q.gs)) return 0;  // its slab constants would not fit in LDS
-  const int lim = env_int("CPQ_SKINNY_MAX_M", 0);  // tuning and test hook
+  const int lim = env_int("CPQ_SKINNY_MAX_M", 0);
   if (lim > 0) return lim;
   return n <= 8192 ? 64 : 32;
 }
@@ -61,15 +59,6 @@ cpq_status launched(hipError_t e, const char* what) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-}  // namespace
-
-// The prefill op on a session: its stream, CU count and fixed-capacity scratch.
-hipError_t launch_session_qmm(cpq_commands* cmds, const QuantArgs& q, const void* x, void* y, int m, int n, int k) {
-  const QmmPlan plan = qmm_plan(q, m, n, k, cmds->dev ? cmds->dev->cu_count : 0, cmds->scratch ? cmds->scratch_bytes : 0);
-  return launch_qmm(cmds->stream, plan, cmds->scratch, q, x, y, m, n, k);
-}
-
-namespace {
 bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }
 
 cpq_status check_ptrs(const char* op, const void* w, const void* s, const void* b, const void* x,
@@ -134,9 +123,10 @@ float small_m_us(const QuantArgs& q, const SmallPlan& sp, bool dense, int m, int
 // 7.8; 16 x 32000 x 1152 13.9 / 16.7; 2 bits, whose slab kernel costs half: 11 x
 // 14752 x 3200 20.9 / 14.7).  4 bits: 2 x 3520 x 3520 6.8 -> 5.0, 8 x
 // 5120 x 2560 9.7 -> 6.9; short rows and, past 4 rows on few columns, K in
-// whole 256s stay (16 x 1152 x 4352 6.4 / 7.1), from 64 blocks on at any
-// rows while K gives a wave a part of its second batch (3 x 1184 x 8448 7.5 / 9.2).  8 bits: 2 x 2560 x 10048 14.5 ->
-// 11.7, 16 x 3520 x 3520 9.9 -> 7.6; many columns stay (32000 x 1152 12.4 / 13.4).
+// whole 256s stay (16 x 1152 x 4352 6.4 / 7.1), from 64 blocks on at any rows
+// while K gives a wave a part of its second batch (3 x 1184 x 8448 7.5 / 9.2).
+// 8 bits: 2 x 2560 x 10048 14.5 -> 11.7, 16 x 3520 x 3520 9.9 -> 7.6; many
+// columns stay (32000 x 1152 12.4 / 13.4).
 bool decode_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
   if (!decode_fits(q, m, n, k, x)) return false;
   const long wgs = (n + 15) / 16;
@@ -147,18 +137,15 @@ bool decode_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
   return k > 1024 && wgs < 1024 && (m <= 4 || k % 256 != 0 || wgs >= 256) && (m <= 8 || k >= 2048 || wgs >= 256);
 }
 
-}  // namespace
-
-namespace {
-
 // Rows that exceed a workgroup's LDS, staged in phases.  Up to 12 rows every
 // wave still has whole batches in LDS, up to K = 12288 in two phases; the grid
 // has to give half the CUs a workgroup and no CU two.  8 x 4096 x 12288 8-bit
 // 24.2 -> 20.0 us, 8 x 3520 x 9984 6-bit 19.8 -> 16.5 and 3-bit 19.1 -> 14.9, 12 x
-// 2048 x 7936 8-bit 16.9 -> 16.2, 8 x 2560 x 10048 4-bit 18.3 -> 13.7.  Others
-// stay: 16 rows (16 x 3520 x 9984 6-bit 20.0 / 22.2), K = 16128 (12 x 2048 6-bit
-// 22.3 / 23.5), 4 bits in whole 256s of K (10 x 3072 x 8448 10.1 / 13.7), 72
-// workgroups (8 x 1152 x 16384 20.7 / 22.8), 768 (8 x 12288 x 4096 19.6 / 24.2).
+// 2048 x 7936 8-bit 16.9 -> 16.2, 8 x 2560 x 10048 4-bit 18.3 -> 13.7.  What
+// stays: K = 16128 (12 x 2048 6-bit 22.1 / 23.3), 768 workgroups (8 x 12288 x
+// 4096 8-bit 18.7 / 23.6), and two classes of which only some lose: 16 rows (16 x
+// 3520 x 9984 6-bit 19.7 / 21.8, but 16 x 3072 x 8448 17.7 / 16.3) and 4 bits in
+// whole 256s of K (10 x 3072 x 8448 9.8 / 13.4, but 12 x 4096 x 12288 19.3 / 16.9).
 bool decode_phased_rows(const QuantArgs& q, int m, int n, int k, const void* x) {
   const long wgs = (n + 15) / 16;
   if (m > 12 || k > 12288 || wgs < 128 || wgs > 256 || (q.bits == 4 && k % 256 == 0)) return false;
@@ -218,7 +205,9 @@ hipError_t launch_matmul(const ExecCtx& ex, const QuantArgs& q, const void* x, v
     const bool dense = dense_ok && small_wgs * 4 < cus;
     const float est = small_m_us(q, sp, dense, m, n, k, cus);
     TilePlan tp{-1, 1, 0, 0.f};
-    if (small_on && dense_env < 1 && est > 6.f) {  // a cheap way out: below it the tiles hardly win (one 64-deep stage takes 4.4)
+    // Below 6 us no look at the tiles: they hardly win there (one 64-deep stage
+    // takes 4.4 us), and the plan costs the host a microsecond.
+    if (small_on && dense_env < 1 && est > 6.f) {
       tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.plan_bytes);
       if (tp.scratch_bytes > ex.scratch_bytes) tp = qmm_tile_t_plan(q, m, n, k, ex.cu_count, ex.scratch_bytes);
     }
