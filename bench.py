@@ -763,8 +763,9 @@ def _pmc_per_dispatch(d, counter):
 
 
 def _short_kernel(name):
-    name = re.sub(r"\((unsigned|cpq::).*$", "", name)
-    return name.replace("void cpq::(anonymous namespace)::", "").replace("cpq::dev::", "")
+    name = name.replace("void ", "", 1).replace("cpq::tile::", "").replace("cpq::dev::", "").replace("cpq::", "")
+    name = name.replace("(anonymous namespace)::", "").replace("> >", ">>")
+    return re.sub(r"\((unsigned|void|cpq::|Args).*$", "", name)
 
 
 def counter_summary(dirs, min_dispatches=20, per_wave=False):
@@ -814,9 +815,9 @@ TRACE_WORKLOADS = (
     ("qmv_lean_kernel<cpq::dev::F16, 4, 6, 4, 4, true, false>", 32768, "cfg1 qmv (f16)"),
     ("qmm_dma_kernel", 131072, "**cfg3a qmm** (headline)"),
     ("qmm_dma_kernel", 196608, "cfg3b"),
-    ("qmm_dma_kernel", 262144, "cfg3c N=4096"),
-    ("qmm_dma_kernel", 786432, "cfg3c N=12288"),
-    ("qmm_tile_t_kernel<cpq::tile::TCfg<cpq::dev::BF16, 8", 65536, "8-bit prefill M=512"),
+    ("TCfg<cpq::dev::BF16, 4, 128, 256", 131072, "cfg3c N=4096"),
+    ("TCfg<cpq::dev::BF16, 4, 128, 256", 393216, "cfg3c N=12288"),
+    ("TCfg<cpq::dev::BF16, 8, 128, 128", 65536, "8-bit prefill M=512"),
     ("qmv_lean_kernel<cpq::dev::BF16, 4, 6, 4, 8, true, false>", 65536, "cfg4 4b gs64 M=1"),
     ("qmv_lean_kernel<cpq::dev::BF16, 4, 5, 4, 8, true, false>", 65536, "cfg4 4b gs32 M=1"),
     ("qmv_lean_kernel<cpq::dev::BF16, 8, 6, 4, 8, true, false>", 65536, "cfg4 8b M=1"),
@@ -836,7 +837,7 @@ TRACE_WORKLOADS = (
     ("gather_decode_kernel<cpq::dev::BF16, 4, 4, true, true>", 77824, "reference qmv gate/up (K=896; dense form, M=1)"),
     ("gather_decode_kernel<cpq::dev::BF16, 4, 4, true, true>", 14336, "reference qmv q/o, its K-padded twin (dense form, M=1)"),
     ("gather_decode_kernel<cpq::dev::BF16, 4, 4, true, true>", 2048, "reference qmv k/v, its K-padded twin (dense form, M=1)"),
-    ("qmv_kernel<cpq::dev::BF16, 4, 8, 4, false>", 28672, "reference qmv down (K=4864)"),
+    ("decode_kernel<cpq::dev::BF16, 4, 6, false>", 35840, "reference qmv down (K=4864)"),
     ("gather_decode_kernel<cpq::dev::BF16, 4, 4, true, true>", 71680, "reference M=39 q, o (K=896) and down (K=4864) (dense form)"),
     ("gather_decode_kernel<cpq::dev::BF16, 4, 4, true, true>", 10240, "reference M=39 k_proj (dense form)"),
     ("gather_decode_kernel<cpq::dev::BF16, 4, 2, true, true>", 194560, "reference M=39 gate/up (dense form)"),

@@ -249,12 +249,12 @@ hipError_t zero_words(hipStream_t s, void* p, size_t n_words) {
 
 // The two-waves-per-SIMD kernel (4-bit, K ranges of whole 1024s) or a tile,
 // whichever is estimated to take less, the first within 3 %; the general kernel
-// for what neither takes.  Measured (4-bit gs64, two-wave kernel / best tile): M = 512, K =
-// 4096: N = 4096 28.9 / 31.6 us, N = 12288 67.5 / 62.8; M = 2048: N = 4096
-// 77.3 / 74.7, N = 12288 226 / 214, N = 4096 at K = 12288 (the two-wave kernel
-// then splits K in 4) 350 / 203.  CPQ_QMM_DMA=0 turns the two-wave kernel off,
-// CPQ_QMM_TILES=0 the tiles; CPQ_QMM_SPLIT forces the K split, on that kernel where it takes it
-// (test hooks, read per call).
+// for what neither takes.  Measured (4-bit gs64, two-wave kernel / best tile):
+// M = 512, K = 4096: N = 4096 26.1 / 30.6 us, N = 12288 65.1 / 64.1; M = 2048:
+// N = 4096 77.3 / 74.7, N = 12288 226 / 214, N = 4096 at K = 12288 (the two-wave
+// kernel then splits K in 4) 350 / 203.  CPQ_QMM_DMA=0 turns the two-wave kernel
+// off, CPQ_QMM_TILES=0 the tiles; CPQ_QMM_SPLIT forces the K split, on that
+// kernel where it takes it (test hooks, read per call).
 QmmPlan qmm_plan(const QuantArgs& q, int m, int n, int k, int cu_count, size_t scratch_cap) {
   const bool sb16 = ((reinterpret_cast<uintptr_t>(q.scales) | reinterpret_cast<uintptr_t>(q.biases)) & 15u) == 0;
   const int forced = env_int("CPQ_QMM_SPLIT", 0);

@@ -8,7 +8,9 @@
 // form of this kernel dequantized into LDS for all waves to read; its LDS
 // traffic (2304 cycles per stage of a 256 x 256 tile against 2048 of MFMA)
 // bounded it.  Here a 256 x 256 tile moves 1280 cycles' worth, and the WM waves
-// of a column block repeat its dequantization: 4.5 VALU per MFMA.
+// of a column block repeat its dequantization.  Counted: 5.9 VALU per MFMA on
+// 128 x 256 tiles at 4 bits (2048 x 12288 x 4096, MFMA busy 51 %), 5.0 on 256 x
+// 256 at 8 bits (777 x 12288 x 4096, 38 %); no LDS bank conflicts.
 #include <algorithm>
 
 #include "qmm_tile.hpp"
